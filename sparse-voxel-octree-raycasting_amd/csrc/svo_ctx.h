@@ -33,6 +33,7 @@ struct svo_ctx {
     uint32_t* d_oct = nullptr;  // validated copy, normal records in breadth-first order
     size_t n_words = 0;
     uint32_t normal_words = 0;  // size of the renumbered normal region
+    bool one_depth = true;      // every normal record is reached at one depth (svo_device_layout)
     uint32_t root = 0;
     int depth = 0;
     // frame buffers

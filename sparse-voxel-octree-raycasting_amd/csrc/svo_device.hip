@@ -38,10 +38,10 @@
 namespace {
 
 constexpr int RAY_BLOCK = 256;
-// Trips per wave-uniform exit check.  Measured on the flythrough (lone
-// ray / warp frames/s / full frames/s): 1: 0.66-0.68 ms / 2,360-2,400 /
-// 880; 2: 0.63 ms / 2,480-2,520 / 920; 4: 0.61-0.63 ms / 2,520-2,560 / 940;
-// 8: 0.60-0.61 ms / 2,530-2,580 / 940-950; 16: the same as 8.
+// Iterations (a step and a descend each) per wave-uniform exit check.
+// Measured on one box (lone ray of 3,589 trips, with 68 us of launch / 1920x1024
+// depth-11 flights: 8 warp frames, 2 full frames): 2: 570 us / 4.51 ms /
+// 1.57 ms; 4: 512 / 4.37 / 1.54; 8: 509 / 4.31 / 1.52; 16: 501 / 4.28 / 1.53.
 #ifndef SVO_TRIP_UNROLL
 #define SVO_TRIP_UNROLL 8
 #endif
@@ -217,10 +217,17 @@ struct Ray {
     float dist, lodsw;
     int ix, iy, iz;
     int rek, lod, sxyz;
-    uint32_t node, before, lroot, test;
+    int qx, qy, qz;  // ray_test: ix, iy, iz >> rek
+    // the last step: changed position bits, their XOR, its level, whether it
+    // was taken as two trips
+    uint32_t any, xd, fuse;
+    int rek0;
+    uint32_t node, lroot;
+    uint32_t ni, st;  // ray_test: child index of the ray's cell, ST_* state
     uint32_t pix;
     uint32_t guard;
-    uint32_t desync;  // nonzero: a step left stale nodes on the stack (no fused trips from then on)
+    uint32_t miss;    // nonzero: ended without a hit (| child_test << 1 of the last trip, trip cap only)
+    int lim;          // pops to rows below it are fused: D, or 0 once a step left stale nodes on the stack
     int view;
     uint32_t blk;  // 8x8 screen block of the ray (long-ray flags of full frames), or NO_BLOCK
 };
@@ -347,136 +354,193 @@ __device__ __forceinline__ int init_ray(Ray& r, uint32_t k, const RayArgs& a)
     r.dist = 0.0f;
     r.lodsw = (float)(V.res_x * 1 * 2);
     r.node = a.root;
-    r.before = a.root;
     r.lroot = 0;
-    r.test = 0;
     r.guard = 0;
-    r.desync = 0u;
+    r.miss = 0u;
+    r.lim = D;
     return RAY_TRACE;
 }
 
 // LDS: node stack, rows 0..D+1 x RAY_BLOCK lanes, then the node cache.
 // Row `rek` (1..D-1) holds the ray's node at depth D-rek; rows D and D+1 hold
 // the root.  So STK(rek) is always the node being tested and STK(rek+1) its
-// parent, and a pop reads both rows without a range check: the reference's
+// parent, and a pop reads its row without a range check: the reference's
 // rows D and D+1 (kernel.cl:635-637) belong to no node of the ray and are
 // read only where they hold the root (rek == D) or where the value is not
 // consulted (a normal depth-1 node's parent, rek == D-1, depths >= 8).
 #define STK(rek) stk[(rek) * RAY_BLOCK + tid]
 constexpr int STK_ROWS_EXTRA = 2;  // rows D and D+1
 
-// One trip of the CAST_RAY do-while loop (kernel.cl:152-211).  Returns true
-// when the loop exits.  A lone wave in the tail of a launch issues one
-// instruction per 4 cycles, so the trip is written for a short path with few
-// exec-mask regions: one divergent branch (descend or step), selects inside
-// each body, the pop as unconditional stack reads at the new level (no pop
-// re-reads the current node and its parent, which the stack also holds), the
-// pop test as one compare (floor(log2 m) >= rek  <=>  m >= 2^rek, m > 0), and
-// the child fetch of fetchChildOffset (kernel.cl:32-62) as one word read.
-template <bool kCache>
-__device__ __forceinline__ uint32_t step_ray(Ray& r, const RayArgs& a, OctBuf ob, uint32_t* stk,
-                                             const uint32_t* cache, int tid)
+// What bounds the trip: a wave issues a vector instruction every 4.5 cycles
+// whether or not it depends on the one before, an exec-mask region costs 44
+// more, a vector compare that a scalar branch waits for 31, an LDS read 52 and
+// an L1 hit 96 (measured on MI355X at 2.4 GHz).  So an iteration has two
+// regions (step, descend) and no branch, flags are 0/1 in vector registers,
+// and what the short path does not cover is left to the end of a group of
+// iterations.  opaque() stops the compiler from turning the flags back into
+// lane masks joined by scalar ands.
+__device__ __forceinline__ uint32_t opaque(uint32_t v)
+{
+    asm("" : "+v"(v));
+    return v;
+}
+
+// r.st of a ray: 0 or 1 (the node has the ray's child cell) while it runs;
+// bit 1: it has ended; bit 2: its last step needs ray_step_rules
+constexpr uint32_t ST_EMPTY = 0, ST_CHILD = 1, ST_ENDED = 2, ST_RULES = 4;
+
+// The child cell of the current node that holds the ray (kernel.cl:152-160):
+// r.ni its index; r.st ST_CHILD when the node has it, with the bits of
+// `flags`.  qx, qy, qz are kept for the step, which needs the same shifts.
+__device__ __forceinline__ void ray_test(Ray& r, uint32_t flags)
+{
+    r.qx = r.ix >> r.rek;
+    r.qy = r.iy >> r.rek;
+    r.qz = r.iz >> r.rek;
+    const uint32_t xy = ((uint32_t)r.qx & 1u) | ((uint32_t)r.qy << 1);
+    const uint32_t xyz = (xy & 3u) | ((uint32_t)r.qz << 2);
+    r.ni = (xyz & 7u) ^ (uint32_t)r.sxyz;
+    r.st = __builtin_amdgcn_ubfe(r.node, r.ni, 1u) | flags;
+}
+
+// Descend trip (kernel.cl:42-61, :169-178): the child word of the node that
+// ray_test found set.  Block nodes address their children from local_root,
+// set on entry from a normal parent; at rek == 2 the depth-(D-1) ref is
+// synthesised from the byte node.  At rek == 1 the fetched word is never
+// consumed (the hit exits and fetchColor reads only the stack).  kTree: every
+// node sits at one depth (all octrees but hand-made ones that share a normal
+// record between depths), so a node is a block node below level 7 and a
+// block's root at level 6; otherwise its own and its parent's block bits say
+// so.  A hit (rek <= lod) leaves the ray at the child: row r.rek is the
+// child, row r.rek + 1 the node that was tested.
+template <bool kCache, bool kTree>
+__device__ __forceinline__ void ray_descend(Ray& r, const RayArgs& a, OctBuf ob, uint32_t* stk, const uint32_t* cache,
+                                            int tid)
+{
+    const int rek = r.rek;
+    const uint32_t node = r.node;
+    const bool blk = kTree ? rek < 7 : (node & 256u) != 0u;
+    const bool enter = kTree ? rek == 6 : blk && !(STK(rek + 1) & 256u);
+    const bool synth = kTree ? rek == 2 : blk && rek == 2;
+    const uint32_t nadd = (uint32_t)__popc(node & ~(~1u << r.ni));
+    const uint32_t n0 = node >> 9;
+    const uint32_t at_root = n0 << 6;
+    const uint32_t in_block = enter ? at_root : n0 + r.lroot;
+    r.lroot = enter ? at_root : r.lroot;
+    const uint32_t off = synth ? (nadd >> 2) : nadd;
+    const uint32_t idx = (blk ? in_block : n0) + (blk ? off : r.ni);
+    uint32_t w;
+    if (kCache && idx < a.cache_words)
+        w = cache[idx];
+    else
+        w = oct_load(ob, idx);
+    const uint32_t byte_ref = __builtin_amdgcn_ubfe(w, nadd << 3, 8u) | ((nadd << 9) | 256u);
+    const uint32_t child = synth ? byte_ref : w;
+    STK(rek - 1) = child;
+    r.node = child;
+    r.rek = rek - 1;
+    r.guard++;
+    ray_test(r, opaque(rek <= r.lod ? ST_ENDED : 0u));
+}
+
+// DDA step trip to the nearest cell face (kernel.cl:181-209), with the
+// reference's next trip fused into it where that trip is known.  After a pop
+// to level nr that left every position bit from nr to D unchanged, the cell
+// at level nr holding the ray is the one it came from: the next trip tests
+// that child, finds it set, and descends into it (kernel.cl:160-179),
+// fetching the ref the stack still holds in row nr-1 -- or stops there as a
+// hit when nr <= lod.  local_root already belongs to that path.  Counted as
+// two trips.
+//
+// The reference pops on the XOR of the three axes' changes, which can sit
+// below the highest changed bit (and bit D is masked out of it).  A step that
+// changed a position bit above the level it resumes at leaves the nodes
+// there, and the stack rows below, describing cells the ray has left; the
+// reference then carries on with those stale nodes, and so does this kernel,
+// but no later step of that ray is fused (r.lim).
+//
+// ray_step takes the common case -- XOR and OR of the changes agree on the
+// level and the ray stays inside the world: with 2^rek - 1 or-ed in, the top
+// bit of the XOR is the row to resume at, or rek - 1 without a pop.  A change
+// of bit D (the world's middle planes and edges, 6% of a flythrough's trips)
+// pops to the root, which the reference reaches through the carry into bit
+// D-1; from the root itself it is no pop.  Anything else -- a change above
+// that row (an XOR-hidden bit, a y crossing), bit D without bit D-1, the far
+// exit -- marks the ray ST_RULES, and ray_step_rules, which states the full
+// rules, then redoes the end of the step (0.15% of the trips).
+constexpr float RAY_FAR = 400000.0f;  // kernel.cl:196
+constexpr uint32_t RAY_FAR_BITS = 0x48c35000u;
+__device__ __forceinline__ void ray_step(Ray& r, const RayArgs& a, const uint32_t* stk, int tid)
+{
+    const int D = a.depth, rek = r.rek;
+    const uint32_t m1 = (1u << rek) - 1u;
+    const float mx = (float)((r.qx + 1) << rek) - r.px;
+    const float my = (float)((r.qy + 1) << rek) - r.py;
+    const float mz = (float)((r.qz + 1) << rek) - r.pz;
+    const float ex = mx * r.lx, ey = my * r.ly, ez = mz * r.lz;
+    const bool c1 = ey < ex;
+    float dist = c1 ? ey : ex;
+    const bool c2 = ez < dist;
+    dist = c2 ? ez : dist;
+    const float m = c2 ? mz : (c1 ? my : mx);
+    const float gx = c2 ? r.g2x : (c1 ? r.g1x : 1.0f);
+    const float gy = c2 ? r.g2y : (c1 ? 1.0f : r.g0y);
+    const float gz = c2 ? 1.0f : (c1 ? r.g1z : r.g0z);
+    r.px += gx * m;
+    r.py += gy * m;
+    r.pz += gz * m;
+    r.dist += dist;
+    const int nx = (int)r.px, ny = (int)r.py, nz = (int)r.pz;
+    const uint32_t cx = (uint32_t)(r.ix ^ nx), cy = (uint32_t)(r.iy ^ ny), cz = (uint32_t)(r.iz ^ nz);
+    r.ix = nx;
+    r.iy = ny;
+    r.iz = nz;
+    // OR and XOR of the changes, bits 0..D (the OR: y also D+1)
+    const uint32_t K1 = (2u << D) - 1u;
+    const uint32_t any = ((cx | cz) & K1) | (cy & (2u * K1 + 1u));
+    const uint32_t xd = ((cx ^ cy ^ cz) & K1) | m1;
+    const int top = 31 - __builtin_clz(xd);
+    const int tm = min(top, D - 1);
+    const uint32_t pop = opaque(tm >= rek ? 1u : 0u);
+    const uint32_t fuse = opaque(top < r.lim ? pop : 0u);
+    const int base = max(tm + 1 - (int)fuse, rek);
+    r.node = STK(base);
+    r.rek = base;
+    // LOD switch, on pops only (kernel.cl:209; a far exit does not pop, but
+    // its LOD is not used again)
+    const uint32_t l = opaque(r.dist > r.lodsw ? pop : 0u);
+    r.lodsw = __builtin_amdgcn_ldexpf(r.lodsw, (int)l);
+    r.lod += (int)l;
+    const uint32_t hit = opaque(base < r.lod ? fuse : 0u);
+    r.guard += fuse + 1u;
+    const uint32_t odd = ((any >> base) & ~1u) | (xd & ~(xd << 1) & (1u << D)) |
+                         ((RAY_FAR_BITS - __float_as_uint(r.dist)) & 0x80000000u);  // sign: beyond RAY_FAR
+    r.any = any;
+    r.xd = xd;
+    r.rek0 = rek;
+    r.fuse = fuse;
+    ray_test(r, (hit << 1) | opaque(odd != 0u ? ST_RULES : 0u));
+}
+
+// the end of a step by the full rules (also of rays near the trip cap)
+__device__ __forceinline__ void ray_step_rules(Ray& r, const RayArgs& a, const uint32_t* stk, int tid)
 {
     const int D = a.depth;
-    const int rek = r.rek;
-    const int p0x = r.ix >> rek, p0y = r.iy >> rek, p0z = r.iz >> rek;
-    const int ni = ((p0x & 1) | ((p0y & 1) << 1) | ((p0z & 1) << 2)) ^ r.sxyz;
-    const uint32_t node = r.node;
-    const uint32_t test = node & (1u << ni);
-    r.test = test;
-    uint32_t done;  // 0/1 as a value (not a lane mask): no mask merges at the join
-    if (test) {
-        // ---- descend (kernel.cl:42-61, :169-178).  Block nodes address their
-        // children from local_root, set on entry from a normal parent; at
-        // rek == 2 the depth-(D-1) ref is synthesised from the byte node.  At
-        // rek == 1 the fetched word is never consumed (the hit exits and
-        // fetchColor reads only node_before and the stack).
-        const uint32_t n0 = node >> 9;
-        const bool blk = (node & 256u) != 0;
-        const bool enter = blk && !(r.before & 256u);
-        const uint32_t lroot = enter ? (n0 << 6) : r.lroot;
-        const uint32_t nadd = (uint32_t)__popc(node & ((test << 1) - 1u));
-        const bool synth = blk && rek == 2;
-        const uint32_t off = synth ? (nadd >> 2) : nadd;
-        const uint32_t idx = (enter ? 0u : n0) + (blk ? lroot + off : (uint32_t)ni);
-        uint32_t w;
-        if (kCache && idx < a.cache_words)
-            w = cache[idx];
-        else
-            w = oct_load(ob, idx);
-        const uint32_t child = synth ? ((w >> ((nadd & 3u) << 3)) & 255u) + 256u + (nadd << 9) : w;
-        r.lroot = lroot;
-        r.before = node;
-        r.node = child;
-        done = (uint32_t)(rek <= r.lod);
-        // the stack write is unconditional: when the ray stops here (rek-1 is
-        // then 0..lod-1) the row is never read again (finish reads row 2 only
-        // for a ray at rek 1, and row 0 never)
-        STK(rek - 1) = child;
-        r.rek = done ? rek : rek - 1;
-    } else {
-        // ---- DDA step to the nearest cell face (kernel.cl:181-194)
-        const float mx = (float)((p0x + 1) << rek) - r.px;
-        const float my = (float)((p0y + 1) << rek) - r.py;
-        const float mz = (float)((p0z + 1) << rek) - r.pz;
-        const float ex = mx * r.lx, ey = my * r.ly, ez = mz * r.lz;
-        const bool c1 = ey < ex;
-        float dist = c1 ? ey : ex;
-        const bool c2 = ez < dist;
-        dist = c2 ? ez : dist;
-        const float m = c2 ? mz : (c1 ? my : mx);
-        const float gx = c2 ? r.g2x : (c1 ? r.g1x : 1.0f);
-        const float gy = c2 ? r.g2y : (c1 ? 1.0f : r.g0y);
-        const float gz = c2 ? 1.0f : (c1 ? r.g1z : r.g0z);
-        r.px += gx * m;
-        r.py += gy * m;
-        r.pz += gz * m;
-        const int nx = (int)r.px, ny = (int)r.py, nz = (int)r.pz;
-        r.dist += dist;
-        // pop level (kernel.cl:197-209): the XOR of the three axes' changes
-        const int DAND = (1 << D) - 1;
-        const int x0ry = r.iy ^ ny;
-        const uint32_t xm = (uint32_t)((r.ix ^ nx) ^ x0ry ^ (r.iz ^ nz)) & (uint32_t)DAND;
-        const uint32_t chg = (uint32_t)((r.ix ^ nx) | x0ry | (r.iz ^ nz)) & ((2u << D) - 1u);  // bits 0..D
-        r.ix = nx;
-        r.iy = ny;
-        r.iz = nz;
-        const bool far = r.dist > 400000.0f;
-        const bool pop = !far && xm >= (1u << rek);
-        const int nr = pop ? 32 - __clz((int)xm) : rek;  // rek_new + 1, or stay
-        // LOD switch, evaluated on pops only (kernel.cl:209)
-        const bool l = pop && r.dist > r.lodsw;
-        r.lodsw = l ? r.lodsw * 2.0f : r.lodsw;
-        r.lod += l ? 1 : 0;
-        const bool ycross = ((uint32_t)x0ry >> (D + 1) & 1u) != 0u;
-        // The reference's next trip, fused into this one.  After a pop to
-        // level nr that left every position bit from nr to D unchanged (the
-        // XOR level can sit below the highest changed bit, and bit D is
-        // masked out of it, so this is checked on the OR of the changes),
-        // the cell at level nr holding the ray is the one it came from: the
-        // next trip tests that child, finds it set, and descends into it
-        // (kernel.cl:160-179), fetching the ref the stack still holds in row
-        // nr-1 -- or stops there as a hit when nr <= lod.  local_root already
-        // belongs to that path.  Counted as two trips; not fused when the
-        // second trip would pass the trip cap.
-        // A step that changed a position bit above the level it resumes at
-        // (the XOR hid it) leaves the nodes there, and the stack rows below,
-        // describing cells the ray has left; the reference then carries on
-        // with those stale nodes, and so does this kernel, but no later
-        // step of the ray is fused.
-        r.desync |= chg >> (nr + 1);
-        const bool fuse = pop && r.desync == 0u && !ycross && (chg >> nr) == 0u && r.guard + 2u <= SVO_MAX_RAY_ITERS;
-        const bool hit = fuse && nr <= r.lod;
-        const int base = fuse ? nr - 1 : nr;
-        r.node = STK(base);
-        r.before = STK(base + 1);
-        r.rek = (fuse && !hit) ? nr - 1 : nr;
-        r.guard += fuse ? 1u : 0u;
-        // a hit's child_test is consumed by fetchColor at level 1 only, and
-        // nr >= 2 here
-        done = (uint32_t)far | (uint32_t)ycross | (uint32_t)hit;
-    }
-    return done;
+    const uint32_t guard = r.guard - r.fuse - 1u;  // before the step
+    const uint32_t xm = r.xd & ((1u << D) - 1u);
+    const uint32_t chg = r.any & ((2u << D) - 1u);
+    const bool ycross = (r.any >> (D + 1)) != 0u;
+    const bool far = r.dist > RAY_FAR;
+    const bool pop = !far && (xm >> r.rek0) != 0u;
+    const int nr = pop ? 32 - __builtin_clz(xm) : r.rek0;
+    if ((chg >> (nr + 1)) != 0u) r.lim = 0;
+    const bool fuse = pop && r.lim != 0 && !ycross && (chg >> nr) == 0u && guard + 2u <= SVO_MAX_RAY_ITERS;
+    const bool hit = fuse && nr <= r.lod;
+    r.rek = fuse ? nr - 1 : nr;
+    r.guard = guard + (fuse ? 2u : 1u);
+    r.miss = (far || ycross) && !hit ? 1u : 0u;
+    r.node = STK(r.rek);
+    ray_test(r, (hit || far || ycross) ? ST_ENDED : 0u);
 }
 
 __device__ __forceinline__ void finish_ray(Ray& r, const RayArgs& a, OctBuf ob, uint32_t* stk, const uint32_t* cache,
@@ -487,8 +551,18 @@ __device__ __forceinline__ void finish_ray(Ray& r, const RayArgs& a, OctBuf ob, 
     if (r.sxyz & 1) px = SCALE_MAX - px;
     if (r.sxyz & 2) py = SCALE_MAX - py;
     if (r.sxyz & 4) pz = SCALE_MAX - pz;
-    uint32_t b2 = (r.rek == 1) ? STK(2) : 0u;
-    uint32_t col = fetch_color(ob, cache, a.cache_words, r.node, r.before, b2, r.lroot, r.rek, r.test);
+    // row r.rek: the child a hit stopped at, or the node a miss left the ray
+    // in; rek is the level whose test ended the ray
+    const int rek = r.rek + (r.miss ? 0 : 1);
+    const uint32_t before = STK(r.rek + 1);
+    uint32_t test = r.miss >> 1, b2 = 0u;
+    if (rek == 1) {
+        b2 = STK(2);
+        if (!r.miss)
+            test = 1u << (((((uint32_t)r.ix >> 1) & 1u) | ((uint32_t)r.iy & 2u) | (((uint32_t)r.iz << 1) & 4u)) ^
+                          (uint32_t)r.sxyz);
+    }
+    uint32_t col = fetch_color(ob, cache, a.cache_words, STK(r.rek), before, b2, r.lroot, rek, test);
     uint32_t word = 0xff000000u + col;
     const View& V = a.views ? a.views[r.view] : a.v;
     V.screen[r.pix] = word;
@@ -511,7 +585,7 @@ __device__ __forceinline__ unsigned long long lane_pattern(int ks)
     return m;
 }
 
-template <bool kCache>
+template <bool kCache, bool kTree>
 __global__ __launch_bounds__(RAY_BLOCK) void k_rays(RayArgs a)
 {
     extern __shared__ uint32_t smem[];
@@ -605,6 +679,7 @@ __global__ __launch_bounds__(RAY_BLOCK) void k_rays(RayArgs a)
                     const int st = init_ray(r, kr, a);
                     active = st == RAY_TRACE;
                     took = st == RAY_MERGED;
+                    if (active) ray_test(r, 0u);
                 }
             }
             traced += (uint32_t)__popcll(__ballot(active)) - (uint32_t)__popcll(~idle_all);
@@ -614,24 +689,39 @@ __global__ __launch_bounds__(RAY_BLOCK) void k_rays(RayArgs a)
             if (exhausted) break;
             continue;
         }
-        // A batch of up to `iters` trips.  Lanes whose ray ends stop (run =
-        // false) and the batch ends early once no lane runs; the loop exit is
-        // wave-uniform, so a trip carries no per-lane loop bookkeeping.  At
-        // most SVO_MAX_RAY_ITERS trips per ray: a ray still running then
-        // finishes at its current node.
-        uint32_t run = active ? 1u : 0u;
+        // A batch of up to `iters` iterations, each a step for the lanes whose
+        // ray is in an empty cell and then a descend for those in a set one,
+        // so a lane may take both (and a fused trip) in one iteration.  Lanes
+        // whose ray ends do neither, and the batch ends early once no lane
+        // runs.  At most SVO_MAX_RAY_ITERS trips per ray: a ray still running
+        // then finishes at its current node (checked once per group, rays
+        // near the cap trip by trip).
+        if (!active) r.st = ST_ENDED;
         for (int it = 0; it < a.iters; it += SVO_TRIP_UNROLL) {
-#pragma unroll
-            for (int u = 0; u < SVO_TRIP_UNROLL; ++u) {
-                if (run) {
-                    const uint32_t d = step_ray<kCache>(r, a, ob, stk, cache, tid);
-                    r.guard++;
-                    run = (d | (uint32_t)(r.guard >= SVO_MAX_RAY_ITERS)) ^ 1u;
+            if (r.st < ST_ENDED && r.guard >= SVO_MAX_RAY_ITERS - 4u * SVO_TRIP_UNROLL) {
+                while (r.st < ST_ENDED) {
+                    const uint32_t bit = r.st == ST_CHILD ? 1u << r.ni : 0u;
+                    if (r.st == ST_CHILD) {
+                        ray_descend<kCache, kTree>(r, a, ob, stk, cache, tid);
+                    } else {
+                        ray_step(r, a, stk, tid);
+                        ray_step_rules(r, a, stk, tid);
+                    }
+                    if (r.st < ST_ENDED && r.guard >= SVO_MAX_RAY_ITERS) {
+                        r.st = ST_ENDED;
+                        r.miss = 1u | (bit << 1);
+                    }
                 }
             }
-            if (__ballot(run != 0u) == 0ull) break;
+#pragma unroll
+            for (int u = 0; u < SVO_TRIP_UNROLL; ++u) {
+                if (r.st == ST_EMPTY) ray_step(r, a, stk, tid);
+                if (__builtin_expect(r.st == ST_CHILD, 1)) ray_descend<kCache, kTree>(r, a, ob, stk, cache, tid);
+            }
+            if (r.st >= ST_RULES) ray_step_rules(r, a, stk, tid);
+            if (__ballot(r.st < ST_ENDED) == 0ull) break;
         }
-        if (active && !run) {
+        if (active && r.st >= ST_ENDED) {
             finish_ray(r, a, ob, stk, cache, tid);
             longest = max(longest, r.guard);
             active = false;
@@ -1316,7 +1406,8 @@ extern "C" int svo_upload_octree(svo_ctx* c, const uint32_t* words, size_t n_wor
     if (n_words < 10 || n_words > (1ull << 29)) return svo_fail(SVO_ERR_ARG, "word count %zu out of range", n_words);
     std::vector<uint32_t> dev;
     uint32_t new_root = 0, normal_words = 0;
-    RC(svo_device_layout(words, n_words, root_ref, depth, dev, &new_root, &normal_words));
+    bool one_depth = true;
+    RC(svo_device_layout(words, n_words, root_ref, depth, dev, &new_root, &normal_words, &one_depth));
     HIPCHECK(hipSetDevice(c->device));
     HIPCHECK(hipStreamSynchronize(c->stream));
     drop_graph(c);
@@ -1330,6 +1421,7 @@ extern "C" int svo_upload_octree(svo_ctx* c, const uint32_t* words, size_t n_wor
     c->root = new_root;
     c->depth = depth;
     c->normal_words = normal_words;
+    c->one_depth = one_depth;
     return SVO_OK;
 }
 
@@ -1632,10 +1724,9 @@ static int launch_rays_v(svo_ctx* c, hipStream_t stream, const View& v, const Vi
         a.split_waves = grid * (unsigned)(RAY_BLOCK / 64) / 2u;
     }
     const size_t lds = ((size_t)(c->depth + STK_ROWS_EXTRA) * RAY_BLOCK + std::max(a.cache_words, 1u)) * 4;
-    if (a.cache_words)
-        hipLaunchKernelGGL(k_rays<true>, dim3(grid), dim3(RAY_BLOCK), lds, stream, a);
-    else
-        hipLaunchKernelGGL(k_rays<false>, dim3(grid), dim3(RAY_BLOCK), lds, stream, a);
+    void (*const kernel)(RayArgs) = c->one_depth ? (a.cache_words ? k_rays<true, true> : k_rays<false, true>)
+                                                 : (a.cache_words ? k_rays<true, false> : k_rays<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(RAY_BLOCK), lds, stream, a);
     HIPCHECK(hipGetLastError());
     return SVO_OK;
 }

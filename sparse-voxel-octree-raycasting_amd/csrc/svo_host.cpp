@@ -379,8 +379,9 @@ struct Validator {
 }  // namespace
 
 int svo_device_layout(const uint32_t* words, size_t n_words, uint32_t root, int depth,
-                      std::vector<uint32_t>& out, uint32_t* new_root, uint32_t* normal_words)
+                      std::vector<uint32_t>& out, uint32_t* new_root, uint32_t* normal_words, bool* one_depth)
 {
+    *one_depth = true;
     const size_t nrec_max = std::min<size_t>(n_words, 2097152) / 10;
     std::vector<int32_t> newidx(nrec_max + 1, -1);
     std::vector<uint32_t> order;
@@ -415,6 +416,8 @@ int svo_device_layout(const uint32_t* words, size_t n_words, uint32_t root, int 
                 newidx[c / 10] = (int32_t)order.size();
                 order.push_back(c);
                 level.push_back(level[q] + 1);
+            } else if (level[newidx[c / 10]] != level[q] + 1) {
+                *one_depth = false;
             }
         }
     }

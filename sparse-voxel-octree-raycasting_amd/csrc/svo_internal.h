@@ -13,9 +13,11 @@ int svo_host_threads();
 
 #include <vector>
 // Validated device copy of a compact word array with the normal region in
-// breadth-first order; *normal_words = size of the renumbered region.
+// breadth-first order; *normal_words = size of the renumbered region;
+// *one_depth = no normal record is reached at two depths (true of every
+// built octree), so a node's depth tells what kind of node it is.
 int svo_device_layout(const uint32_t* words, size_t n_words, uint32_t root, int depth,
-                      std::vector<uint32_t>& out, uint32_t* new_root, uint32_t* normal_words);
+                      std::vector<uint32_t>& out, uint32_t* new_root, uint32_t* normal_words, bool* one_depth);
 
 // Hard bound on traversal iterations per ray (a ray that has not exited
 // after this many loop trips is finished as a miss at its current node).
