@@ -90,3 +90,67 @@ def test_trip_cap():
         c.raycast_rect(p, 7, 7, 2, 1)
         c.sync()
         assert c.ray_stats() == (2, 1 << 22)
+
+
+@pytest.mark.parametrize("wg", [1, 5])
+@pytest.mark.parametrize("lanes", [1, 8, 64])
+@pytest.mark.parametrize("group", [1, 64])
+def test_hand_out(wg, lanes, group):
+    """Each ray is handed out once, in launches with fewer waves of rays than
+    the grid has, as many, and more (1 lane per wave): full frames (long
+    blocks from the second on) and warp frames, ray counts included."""
+    words, root = scene_octree(CONFIG1["kind"], CONFIG1["seed"], CONFIG1["depth"])
+    rx, ry = 131, 67
+    pr = path(CONFIG1, 5)
+    o = O.Frame(rx, ry, words, root, 8, nthreads=8)
+    with S.Context(0) as c:
+        c.upload_octree(words, root, 8)
+        c.resize(rx, ry)
+        c.set_tuning(wg_per_cu=wg, refill=3, iters=16)
+        c.set_ray_lanes(lanes)
+        c.set_ray_spread(group, only_if_fits=False)
+        c.set_long_first(300)
+        c.set_pretrace(sets=0)
+        for f in range(4):
+            p = params(CONFIG1, pr, f)
+            print(f"wg {wg} lanes {lanes} group {group} frame {f}", flush=True)
+            c.ray_stats(reset=True)
+            c.frame_warp(p)
+            o.frame_warp(O.params_from(p))
+            assert_equal_u32(c.screen(), o.screen, f"warp frame {f}")
+            assert c.ray_count(reset=True) == c.hole_count() + rect_pixels(rx, ry, f)
+        full = O.Frame(rx, ry, words, root, 8, nthreads=8)
+        for f in range(2):
+            p = params(CONFIG1, pr, f)
+            c.ray_stats(reset=True)
+            c.frame_full(p)
+            full.frame_full(O.params_from(p))
+            assert_equal_u32(c.screen(0), full.screen[0], f"full frame {f}")
+            assert c.ray_count() == rx * ry
+        full.close()
+    o.close()
+
+
+def rect_pixels(rx, ry, f):
+    ax, ay, ex, ey = S.tile_schedule(rx, ry, f)
+    return max(0, min(ax + ex, rx) - ax) * max(0, min(ay + ey, ry) - ay)
+
+
+@pytest.mark.parametrize("n", [(1, 1), (8, 8), (9, 8), (64, 63), (131, 67)])
+def test_rect_sizes(n):
+    """Rectangles from one ray to the screen: pixels inside are the oracle's,
+    the others keep the hole word, and each ray is counted once."""
+    words, root = scene_octree(CONFIG1["kind"], CONFIG1["seed"], CONFIG1["depth"])
+    rx, ry = 131, 67
+    p = params(CONFIG1, path(CONFIG1, 1), 0)
+    ref = oracle(words, root, 8, p, (rx, ry))[0]
+    want = np.full((ry, rx), S.HOLE, np.uint32)
+    want[:n[1], :n[0]] = ref[:n[1], :n[0]]
+    with S.Context(0) as c:
+        c.upload_octree(words, root, 8)
+        c.resize(rx, ry)
+        c.memset(0, S.HOLE, 4 * c.N)
+        print(f"rect {n}", flush=True)
+        c.raycast_rect(p, 0, 0, *n)
+        assert_equal_u32(c.screen(0), want, "screen")
+        assert c.ray_count() == n[0] * n[1]
