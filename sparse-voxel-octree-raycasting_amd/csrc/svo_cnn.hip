@@ -37,17 +37,6 @@ __device__ __forceinline__ bf16 f2bf(float f)
     return (bf16)(u >> 16);
 }
 __device__ __forceinline__ float bf2f(bf16 h) { return __uint_as_float((uint32_t)h << 16); }
-// relu(acc + bias) of four channels as four bf16 (channel 0 in the low half)
-__device__ __forceinline__ uint2 relu_bf16x4(f4v acc, f4v bias)
-{
-    uint32_t h[4];
-    for (int i = 0; i < 4; i++) {
-        const float v = acc[i] + bias[i];
-        h[i] = (uint32_t)f2bf(v > 0.f ? v : 0.f);
-    }
-    return make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-}
-
 constexpr uint32_t HOLE_WORD = 0xffffff00u;
 constexpr int TILE = 8;          // output tile edge per wave
 constexpr int HALO = TILE + 2;   // input tile edge
@@ -388,23 +377,54 @@ __global__ __launch_bounds__(256) void k_cnn_apply(const uint32_t* __restrict__ 
 // 16x16 gate tile, activations in LDS.  Each layer is evaluated only where
 // the centre 16x16 output needs it: layer 1 on 22x22, layer 2 on 20x20,
 // layer 3 on 18x18, layer 4 on 16x16 (the crop border's zero padding never
-// reaches the centre, so this equals the full-crop network there).  An
-// M-tile is 16 consecutive output pixels in raster order; layer 1 uses
-// v_mfma_f32_16x16x16_bf16 over K = 16 channels per tap, layers 2-4
-// v_mfma_f32_16x16x32_bf16 over K = 32 (A lane: pixel l%16, channels
-// 8*(l/16)..+7; B lane: output channel l%16, the same 8 input channels).
+// reaches the centre, so this equals the full-crop network there).  Layer 1
+// uses v_mfma_f32_16x16x16_bf16 over K = 16 channels per tap, layers 2-4
+// v_mfma_f32_16x16x32_bf16 over K = 32 (lane: pixel or output channel l%16,
+// input channels 8*(l/16)..+7).
+//
+// Three resources bound a tile: the matrix cores (1,584 MFMAs of 16 cycles
+// over 4 SIMDs), the LDS reads of the pixel fragments, and the vector
+// instructions around them (addresses, bias, ReLU, bf16).  An M-tile per 16
+// consecutive pixels reads nine fragments per pair of output channel groups
+// and computes nine swizzled addresses.  Here a wave sweeps a band of rows of
+// the leftmost 16 columns: each input row's three fragments (dx = 0..2) feed
+// the three output rows they belong to, so a row costs three reads instead of
+// nine, from three addresses per layer with the row as the instruction's
+// offset.  The remaining columns (6, 4 and 2 of layers 1-3) are M-tiles of 16
+// pixels each, a wave's M-tiles of a layer computed together.  Every output
+// adds its taps 0..8 in that order.  A wave computes 16 of the hidden layers'
+// 32 output channels, so layers 1-3's weights stay in its registers for the
+// whole launch (layer 4's come from the L2 behind layer 3), a tile has four
+// barriers, and the next tile's crop is on its way from memory during layers
+// 3 and 4.  6,250 tiles of a 1920x1024 learned frame, stage time with nothing
+// beside it on one device: 276.5 us with nine reads per M-tile and each
+// layer's weights staged in LDS, 203 with the sweep and the resident weights,
+// 178 with the next row's fragments read behind a row's first MFMAs, 169 with
+// layer 4's RGB stored from its registers and the crop fetched ahead.  At 169
+// the matrix cores are busy 39 % of the time; two waves per SIMD (LDS and
+// registers both allow no more) leave each other's stalls uncovered.
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 
-// 32-channel pixels: the 16-byte channel group g of pixel p sits in slot
-// g ^ ((p >> 1) & 3).  A 128-bit LDS read is served 8 lanes at a time from
-// 128 bytes of banks: 8 consecutive pixels (64-byte stride) of one group
-// then land on 8 distinct 16-byte bank slots (pixel parity x slot)
-__device__ __forceinline__ int swz(int p, int g) { return p * 32 + ((g ^ ((p >> 1) & 3)) << 3); }
-// 16-channel input pixels (layer 1): the 8-byte group k (4 channels) of
-// pixel p sits in slot k ^ ((p >> 2) & 3); a 64-bit read is served 16 lanes
-// at a time from 128 bytes, and 16 consecutive pixels (32-byte stride) of
+// 32-channel buffers: rows of TILE_PITCH pixels of 64 bytes; the 16-byte
+// channel group g of column x sits in slot g ^ ((x >> 1) & 3).  A 128-bit LDS
+// read is served 8 lanes at a time from 128 bytes of banks: 8 consecutive
+// columns of one group then land on 8 distinct 16-byte slots (column parity x
+// slot).  The slot depends on the column alone, so a row further down is a
+// constant offset; the odd pitch shifts the next row by half of the banks,
+// which spreads M-tiles of several short rows.
+constexpr int TILE_PITCH = 25;
+__device__ __forceinline__ int at32(int y, int x, int g)
+{
+    return (y * TILE_PITCH + x) * 32 + ((g ^ ((x >> 1) & 3)) << 3);
+}
+// the 24x24 input, 16-channel pixels: the 8-byte group k (4 channels) of
+// column x sits in slot k ^ ((x >> 2) & 3); a 64-bit read is served 16 lanes
+// at a time from 128 bytes, and 16 consecutive columns (32-byte stride) of
 // one group then cover 16 distinct 8-byte slots
-__device__ __forceinline__ int swz1(int p, int k) { return p * 16 + ((k ^ ((p >> 2) & 3)) << 2); }
+__device__ __forceinline__ int at16(int y, int x, int k)
+{
+    return (y * 24 + x) * 16 + ((k ^ ((x >> 2) & 3)) << 2);
+}
 
 // One view's CNN tiles in frame mode: features of the crop at tile*16 - 4
 // from the view's CNN input planes, 256 colorized words per tile to `staged`;
@@ -464,217 +484,303 @@ __global__ __launch_bounds__(256) void k_cnn_apply_views(const TileView* views)
     }
 }
 
-// Both tile layers compute the transposed product D[channel][pixel] (the
-// weights are the MFMA's A operand, the pixels its B operand), so a lane
-// ends with four consecutive output channels of one pixel and stores them as
-// one 8-byte write.
+// All tile layers compute the transposed product D[channel][pixel] (the
+// weights are the MFMA's A operand, the pixels its B operand), so a lane ends
+// with four consecutive output channels of one pixel and stores them as one
+// 8-byte write.
 
-// layers 2-4: in = swizzled 32-channel pixels of a win x win region, Wl =
-// swizzled [9][COUT][32] weights
-template <int COUT, bool LAST>
-__device__ __forceinline__ void tile_layer32(const bf16* in, int win, bf16* out, float* outf, int wout,
-                                             const bf16* Wl, const float* __restrict__ bias, int wave, int lane,
-                                             int nw)
+// relu(acc + bias) of four channels as four bf16 (round to nearest even, as f2bf)
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint2 relu_pack(f4v acc, f4v bias)
 {
-    constexpr int NT = COUT / 16;
-    const int npix = wout * wout;
-    const int row = lane & 15, kg = lane >> 4;
-    // the layer's B fragments stay in registers for all of the wave's M-tiles
-    bf8v bfr[9][NT];
-    for (int tap = 0; tap < 9; tap++)
-        for (int nn = 0; nn < NT; nn++) bfr[tap][nn] = *(const bf8v*)(Wl + swz(tap * COUT + nn * 16 + row, kg));
-    // this lane's output channels: nn * 16 + kg * 4 + i
-    f4v bv[NT];
-    for (int nn = 0; nn < NT; nn++)
-        for (int i = 0; i < 4; i++) bv[nn][i] = bias[nn * 16 + kg * 4 + i];
-    for (int m0 = wave * 2; m0 * 16 < npix; m0 += 2 * nw) {
-        f4v acc[2][NT];
-        int q0[2];
-        for (int m = 0; m < 2; m++) {
-            for (int nn = 0; nn < NT; nn++) acc[m][nn] = f4v{0.f, 0.f, 0.f, 0.f};
-            const int p = min((m0 + m) * 16 + row, npix - 1);  // past the end: recomputed, not stored
-            q0[m] = (p / wout) * win + p % wout;
-        }
-        for (int tap = 0; tap < 9; tap++) {
-            const int dq = (tap / 3) * win + tap % 3;
-            for (int m = 0; m < 2; m++) {
-                const bf8v afr = *(const bf8v*)(in + swz(q0[m] + dq, kg));
-                for (int nn = 0; nn < NT; nn++)
-                    acc[m][nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[tap][nn], afr, acc[m][nn], 0, 0, 0);
+    f4v v = acc + bias;
+    for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i], 0.f);
+    union {
+        bf2v h[2];
+        uint2 u;
+    } o;
+    o.h[0] = __builtin_convertvector(f2v{v[0], v[1]}, bf2v);
+    o.h[1] = __builtin_convertvector(f2v{v[2], v[3]}, bf2v);
+    return o.u;
+}
+
+// one layer's weights and biases of a wave's 16 output channels: fragment
+// [tap] = this lane's output channel and input channels; bias of the 4
+// channels it ends with
+template <typename Frag>
+struct TileWeights {
+    Frag w[9];
+    f4v b;
+    // W: [9][cout][cin], the channels from co0 on
+    __device__ __forceinline__ void load(const bf16* __restrict__ W, const float* __restrict__ bias, int cout, int cin,
+                                         int co0, int row, int kg)
+    {
+#pragma unroll
+        for (int t = 0; t < 9; t++)
+            w[t] = *(const Frag*)(W + (t * cout + co0 + row) * cin + kg * (int)(sizeof(Frag) / 2));
+        b = *(const f4v*)(bias + co0 + kg * 4);
+    }
+};
+
+__device__ __forceinline__ f4v tile_mfma(s4v w, s4v x, f4v acc)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(w, x, acc, 0, 0, 0);
+}
+__device__ __forceinline__ f4v tile_mfma(bf8v w, bf8v x, f4v acc)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, acc, 0, 0, 0);
+}
+
+// fragment address of input pixel (y, x): 16-channel input or 32-channel buffer
+__device__ __forceinline__ int tile_at(s4v, int y, int x, int kg) { return at16(y, x, kg); }
+__device__ __forceinline__ int tile_at(bf8v, int y, int x, int kg) { return at32(y, x, kg); }
+template <typename Frag>
+constexpr int tile_row_step()
+{
+    return sizeof(Frag) == 8 ? 24 * 16 : TILE_PITCH * 32;
+}
+
+// ROWS output rows from y0 on, columns 0..15: acc[r]
+template <int ROWS, typename Frag>
+__device__ __forceinline__ void tile_sweep(const bf16* in, int y0, const TileWeights<Frag>& W, int row, int kg,
+                                           f4v (&acc)[ROWS])
+{
+    const bf16* base[3];
+    for (int dx = 0; dx < 3; dx++) base[dx] = in + tile_at(Frag(), y0, row + dx, kg);
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) acc[r] = f4v{0.f, 0.f, 0.f, 0.f};
+    // the next row's fragments are read behind this row's first three MFMAs
+    Frag f[2][3];
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++) f[0][dx] = *(const Frag*)base[dx];
+#pragma unroll
+    for (int j = 0; j < ROWS + 2; j++) {
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) {
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+                const int r = j - dy;
+                if (r >= 0 && r < ROWS) acc[r] = tile_mfma(W.w[dy * 3 + dx], f[j & 1][dx], acc[r]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (dx == 0 && j + 1 < ROWS + 2) {
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+                    f[(j + 1) & 1][d] = *(const Frag*)(base[d] + (j + 1) * tile_row_step<Frag>());
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        for (int m = 0; m < 2; m++) {
-            const int q = (m0 + m) * 16 + row;
-            if (q >= npix) continue;
-            for (int nn = 0; nn < NT; nn++) {
-                const int co0 = nn * 16 + kg * 4;
-                if (LAST) {
-                    if (co0 == 0)
-                        for (int i = 0; i < 3; i++) outf[q * 3 + i] = acc[m][nn][i] + bv[nn][i];
+    }
+}
+
+// a hidden layer: EDGE x EDGE output pixels (EDGE - 16 columns beside the
+// swept 16) from `in` into the 32-channel buffer `out`; wave w computes
+// channels 16 * (w & 1) .. + 15 of half of the rows (w >> 1) and of every
+// second M-tile of the other columns
+template <int EDGE, typename Frag>
+__device__ __forceinline__ void tile_layer(const bf16* in, bf16* out, const TileWeights<Frag>& W, int wave, int lane)
+{
+    constexpr int ROWS = EDGE / 2;
+    asm volatile("" : "+v"(lane));  // the addresses are computed here, not kept in registers across tiles
+    const int row = lane & 15, kg = lane >> 4, band = wave >> 1, y0 = band * ROWS;
+    const int g = (wave & 1) * 2 + (kg >> 1), gofs = (kg & 1) * 4;  // this lane's 4 output channels
+    f4v acc[ROWS];
+    tile_sweep<ROWS>(in, y0, W, row, kg, acc);
+    bf16* o = out + at32(y0, row, g) + gofs;
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) *(uint2*)(o + r * TILE_PITCH * 32) = relu_pack(acc[r], W.b);
+    // its M-tiles band, band + 2, ... of the other columns together, so their
+    // chains of nine dependent MFMAs overlap
+    constexpr int RC = EDGE - 16, CNT = EDGE * RC, NM = ((CNT + 15) / 16 + 1) / 2;
+    const bf16* base[NM][3];
+    f4v c[NM];
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+        const int i = min((band + 2 * m) * 16 + row, CNT - 1);  // past the end: the last pixel again, not stored
+        for (int dx = 0; dx < 3; dx++) base[m][dx] = in + tile_at(Frag(), i / RC, 16 + i % RC + dx, kg);
+        c[m] = f4v{0.f, 0.f, 0.f, 0.f};
+    }
+    Frag f[2][NM];
+#pragma unroll
+    for (int m = 0; m < NM; m++) f[0][m] = *(const Frag*)base[m][0];
+#pragma unroll
+    for (int tap = 0; tap < 9; tap++) {
+        if (tap < 8)
+#pragma unroll
+            for (int m = 0; m < NM; m++)
+                f[(tap + 1) & 1][m] =
+                    *(const Frag*)(base[m][(tap + 1) % 3] + (tap + 1) / 3 * tile_row_step<Frag>());
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < NM; m++) c[m] = tile_mfma(W.w[tap], f[tap & 1][m], c[m]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+        const int i = (band + 2 * m) * 16 + row;
+        if (i < CNT) *(uint2*)(out + at32(i / RC, 16 + i % RC, g) + gofs) = relu_pack(c[m], W.b);
+    }
+}
+
+// The crop of tile c, pixels tid, tid + 256, tid + 512 of its 576: read from
+// memory into registers (fetch), then features into the LDS input (put).
+template <bool kExplicit>
+struct TileCrop {  // frame mode: screen word and position
+    uint32_t word[3];
+    float px[3], py[3], pz[3];
+    bool in[3];  // inside the screen
+};
+template <>
+struct TileCrop<true> {
+    uint4 lo[3], hi[3];
+};
+
+__device__ __forceinline__ const TileView* tile_view_of(const TileArgs& a, int c, int& lc)
+{
+    lc = c;
+    if (!a.views) return &a.v;
+    int lo = 0, hi = a.n_views - 1;  // the last view whose first tile is <= c
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if ((int)a.first[mid] <= c) lo = mid;
+        else hi = mid - 1;
+    }
+    lc = c - (int)a.first[lo];
+    return &a.views[lo];
+}
+
+__device__ __forceinline__ void tile_fetch(const TileArgs& a, int c, int tid, TileCrop<true>& q)
+{
+    asm volatile("" : "+v"(tid));  // as in tile_layer
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int p = min(tid + 256 * k, 575);
+        const uint4* src = (const uint4*)(a.x + ((size_t)c * 576 + p) * 16);
+        q.lo[k] = src[0];
+        q.hi[k] = src[1];
+    }
+}
+
+__device__ __forceinline__ void tile_fetch(const TileArgs& a, int c, int tid, TileCrop<false>& q)
+{
+    asm volatile("" : "+v"(tid));  // as in tile_layer
+    int lc;
+    const TileView* V = tile_view_of(a, c, lc);
+    const int t = (int)V->tiles[lc];
+    const int ox = (t % V->tiles_x) * 16 - 4, oy = (t / V->tiles_x) * 16 - 4;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int p = tid + 256 * k;
+        const int x = ox + p % 24, y = oy + p / 24;
+        q.in[k] = p < 576 && x >= 0 && y >= 0 && x < V->res_x && y < V->res_y;
+        if (!q.in[k]) continue;
+        const size_t o = (size_t)y * V->res_x + x;
+        q.word[k] = V->words[o];
+        const float4 pos = V->coords[o];
+        q.px[k] = pos.x;
+        q.py[k] = pos.y;
+        q.pz[k] = pos.z;
+    }
+}
+
+__device__ __forceinline__ void tile_put(const TileArgs&, int, int tid, const TileCrop<true>& q, bf16* P)
+{
+    asm volatile("" : "+v"(tid));
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int p = tid + 256 * k, y = p / 24, x = p % 24;
+        if (p >= 576) continue;
+        *(uint2*)(P + at16(y, x, 0)) = make_uint2(q.lo[k].x, q.lo[k].y);
+        *(uint2*)(P + at16(y, x, 1)) = make_uint2(q.lo[k].z, q.lo[k].w);
+        *(uint2*)(P + at16(y, x, 2)) = make_uint2(q.hi[k].x, q.hi[k].y);
+        *(uint2*)(P + at16(y, x, 3)) = make_uint2(q.hi[k].z, q.hi[k].w);
+    }
+}
+
+__device__ __forceinline__ void tile_put(const TileArgs& a, int c, int tid, const TileCrop<false>& q, bf16* P)
+{
+    asm volatile("" : "+v"(tid));
+    int lc;
+    const TileView* V = tile_view_of(a, c, lc);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int p = tid + 256 * k, y = p / 24, x = p % 24;
+        if (p >= 576) continue;
+        float f[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+        if (q.in[k]) {
+            if (q.word[k] == HOLE_WORD) {
+                f[4] = 1.f;
+            } else {
+                rgb_of(q.word[k], f[0], f[1], f[2]);
+                const float qx = q.px[k] - V->m0x, qy = q.py[k] - V->m0y, qz = q.pz[k] - V->m0z;
+                const float z = fmaxf((qx * V->r20 + qy * V->r21) + qz * V->r22, 0.f);
+                f[3] = z / (z + 64.f);
+            }
+        }
+        *(uint2*)(P + at16(y, x, 0)) = make_uint2((uint32_t)f2bf(f[0]) | ((uint32_t)f2bf(f[1]) << 16),
+                                                  (uint32_t)f2bf(f[2]) | ((uint32_t)f2bf(f[3]) << 16));
+        *(uint2*)(P + at16(y, x, 1)) = make_uint2((uint32_t)f2bf(f[4]), 0u);
+        *(uint2*)(P + at16(y, x, 2)) = make_uint2(0u, 0u);
+        *(uint2*)(P + at16(y, x, 3)) = make_uint2(0u, 0u);
+    }
+}
+
+// LDS pixels of the 32-channel buffers (the last row ends at its last column)
+constexpr int tile_pixels(int edge) { return (edge - 1) * TILE_PITCH + edge; }
+
+// two waves per SIMD: 256 registers each, the weights need 99 of them
+template <bool kExplicit>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_cnn_tiles(TileArgs a)
+{
+    __shared__ __align__(16) bf16 P[tile_pixels(20) * 32];  // the 24x24 input, then layer 2's output
+    __shared__ __align__(16) bf16 Q[tile_pixels(22) * 32];  // layer 1's output, then layer 3's
+    static_assert(576 * 16 <= tile_pixels(20) * 32, "the input fits in P");
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, row = lane & 15, kg = lane >> 4;
+    const int n = kExplicit ? a.n : a.views ? (int)a.first[a.n_views] : min((int)*a.v.count, a.v.max_tiles);
+    int c = blockIdx.x;
+    if (c >= n) return;
+    const int co0 = (wave & 1) * 16;  // this wave's channels of the hidden layers
+    TileWeights<s4v> w1;
+    TileWeights<bf8v> w2, w3;
+    w1.load(a.w[0], a.b[0], 32, 16, co0, row, kg);
+    w2.load(a.w[1], a.b[1], 32, 32, co0, row, kg);
+    w3.load(a.w[2], a.b[2], 32, 32, co0, row, kg);
+    TileCrop<kExplicit> crop;
+    tile_fetch(a, c, tid, crop);
+    for (; c < n; c += gridDim.x) {
+        tile_put(a, c, tid, crop, P);  // every wave is past layer 3 of the tile before: P is free
+        __syncthreads();
+        tile_layer<22>(P, Q, w1, wave, lane);
+        __syncthreads();
+        tile_layer<20>(Q, P, w2, wave, lane);
+        __syncthreads();
+        if (c + (int)gridDim.x < n) tile_fetch(a, c + gridDim.x, tid, crop);
+        // layer 4's weights are read again per tile: 36 more registers would spill
+        const bf16* w4p = a.w[3];
+        asm volatile("" : "+s"(w4p));
+        TileWeights<bf8v> w4;
+        w4.load(w4p, a.b[3], 16, 32, 0, row, kg);
+        tile_layer<18>(P, Q, w3, wave, lane);
+        __syncthreads();
+        // layer 4: RGB are the first channels, held by the lanes of kg 0
+        f4v acc[4];
+        tile_sweep<4>(Q, wave * 4, w4, row, kg, acc);
+        if (kg == 0) {
+            int lc;
+            const TileView* V = tile_view_of(a, c, lc);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const f4v v = acc[r] + w4.b;
+                const int px = (wave * 4 + r) * 16 + row;
+                if (kExplicit) {
+                    float* o = a.out + ((size_t)c * 256 + px) * 3;
+                    o[0] = v[0];
+                    o[1] = v[1];
+                    o[2] = v[2];
                 } else {
-                    *(uint2*)(out + swz(q, co0 >> 3) + (co0 & 7)) = relu_bf16x4(acc[m][nn], bv[nn]);
+                    V->staged[(size_t)lc * 256 + px] = rgb_word(v[0], v[1], v[2]);
                 }
-            }
-        }
-    }
-}
-
-// weights of the four layers as the tile kernel keeps them in LDS: layer 1
-// [9][32][16] plain, layers 2-4 [9][COUT][32] with swizzled rows
-constexpr int W_OFS1 = 9 * 32 * 16, W_OFS2 = W_OFS1 + 9 * 32 * 32, W_OFS3 = W_OFS2 + 9 * 32 * 32;
-constexpr int W_ALL = W_OFS3 + 9 * 16 * 32;
-
-__device__ __forceinline__ void stage_weights(bf16* dst, const bf16* __restrict__ src, int rows, bool swizzled,
-                                              int tid, int nthreads)
-{
-    if (!swizzled) {
-        for (int i = tid; i < rows * 16 / 8; i += nthreads) *(uint4*)(dst + i * 8) = *(const uint4*)(src + i * 8);
-        return;
-    }
-    for (int i = tid; i < rows * 4; i += nthreads) {
-        const int r = i >> 2, g = i & 3;
-        *(uint4*)(dst + swz(r, g)) = *(const uint4*)(src + r * 32 + g * 8);
-    }
-}
-
-// layer 1: 16 -> 32 on 22x22 from the 24x24 plain 16-channel input
-__device__ __forceinline__ void tile_layer1(const bf16* P, bf16* Q, const bf16* Wl, const float* __restrict__ bias,
-                                            int wave, int lane, int nw)
-{
-    const int row = lane & 15, kg = lane >> 4;
-    s4v b1[9][2];
-    for (int tap = 0; tap < 9; tap++)
-        for (int nn = 0; nn < 2; nn++) b1[tap][nn] = *(const s4v*)(Wl + (tap * 32 + nn * 16 + row) * 16 + kg * 4);
-    f4v bv[2];
-    for (int nn = 0; nn < 2; nn++)
-        for (int i = 0; i < 4; i++) bv[nn][i] = bias[nn * 16 + kg * 4 + i];
-    for (int m0 = wave * 2; m0 * 16 < 484; m0 += 2 * nw) {
-        f4v acc[2][2];
-        int q0[2];
-        for (int m = 0; m < 2; m++) {
-            acc[m][0] = acc[m][1] = f4v{0.f, 0.f, 0.f, 0.f};
-            const int p = min((m0 + m) * 16 + row, 483);
-            q0[m] = (p / 22) * 24 + p % 22;
-        }
-        for (int tap = 0; tap < 9; tap++) {
-            const int dq = (tap / 3) * 24 + tap % 3;
-            for (int m = 0; m < 2; m++) {
-                const s4v afr = *(const s4v*)(P + swz1(q0[m] + dq, kg));
-                for (int nn = 0; nn < 2; nn++)
-                    acc[m][nn] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(b1[tap][nn], afr, acc[m][nn], 0, 0, 0);
-            }
-        }
-        for (int m = 0; m < 2; m++) {
-            const int q = (m0 + m) * 16 + row;
-            if (q >= 484) continue;
-            for (int nn = 0; nn < 2; nn++) {
-                const int co0 = nn * 16 + kg * 4;
-                *(uint2*)(Q + swz(q, co0 >> 3) + (co0 & 7)) = relu_bf16x4(acc[m][nn], bv[nn]);
-            }
-        }
-    }
-}
-
-// NW waves per workgroup.  RESIDENT: the four layers' weights are staged in
-// LDS once per workgroup (8 waves, one workgroup per CU); otherwise each
-// layer's weights are staged per tile (4 waves, two workgroups per CU).
-template <int NW, bool RESIDENT>
-__global__ __launch_bounds__(NW * 64) void k_cnn_tiles(TileArgs a)
-{
-    __shared__ __align__(16) bf16 P[400 * 32];  // input 576 x 16 ch / layer-2 output 400 x 32 ch / layer-4 RGB
-    __shared__ __align__(16) bf16 Q[484 * 32];  // layer-1 output 484 x 32 / layer-3 output 324 x 32
-    __shared__ __align__(16) bf16 Wl[RESIDENT ? W_ALL : 9 * 32 * 32];
-    float* OF = (float*)P;  // 256 x 3 floats, written by layer 4 after layer 3 has consumed P
-    constexpr int NT = NW * 64;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int n = a.x ? a.n : a.views ? (int)a.first[a.n_views] : min((int)*a.v.count, a.v.max_tiles);
-    if (RESIDENT) {
-        stage_weights(Wl, a.w[0], 9 * 32, false, tid, NT);
-        stage_weights(Wl + W_OFS1, a.w[1], 9 * 32, true, tid, NT);
-        stage_weights(Wl + W_OFS2, a.w[2], 9 * 32, true, tid, NT);
-        stage_weights(Wl + W_OFS3, a.w[3], 9 * 16, true, tid, NT);
-    }
-    for (int c = blockIdx.x; c < n; c += gridDim.x) {
-        __syncthreads();  // the previous crop is done with every buffer (and the weights are staged)
-        int ox = 0, oy = 0, lc = c;
-        const TileView* V = &a.v;
-        if (a.views) {  // the last view whose first tile is <= c
-            int lo = 0, hi = a.n_views - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if ((int)a.first[mid] <= c) lo = mid;
-                else hi = mid - 1;
-            }
-            V = &a.views[lo];
-            lc = c - (int)a.first[lo];
-        }
-        if (!a.x) {
-            const int t = (int)V->tiles[lc];
-            ox = (t % V->tiles_x) * 16 - 4;
-            oy = (t / V->tiles_x) * 16 - 4;
-        }
-        for (int q = tid; q < 576; q += NT) {
-            uint4 lo = make_uint4(0u, 0u, 0u, 0u), hi = lo;
-            if (a.x) {
-                const uint4* src = (const uint4*)(a.x + ((size_t)c * 576 + q) * 16);
-                lo = src[0];
-                hi = src[1];
-            } else {
-                const int x = ox + q % 24, y = oy + q / 24;
-                float f[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
-                if (x >= 0 && y >= 0 && x < V->res_x && y < V->res_y) {
-                    const size_t o = (size_t)y * V->res_x + x;
-                    const uint32_t w = V->words[o];
-                    if (w == HOLE_WORD) {
-                        f[4] = 1.f;
-                    } else {
-                        rgb_of(w, f[0], f[1], f[2]);
-                        const float4 cc = V->coords[o];
-                        const float qx = cc.x - V->m0x, qy = cc.y - V->m0y, qz = cc.z - V->m0z;
-                        const float z = fmaxf((qx * V->r20 + qy * V->r21) + qz * V->r22, 0.f);
-                        f[3] = z / (z + 64.f);
-                    }
-                }
-                lo.x = (uint32_t)f2bf(f[0]) | ((uint32_t)f2bf(f[1]) << 16);
-                lo.y = (uint32_t)f2bf(f[2]) | ((uint32_t)f2bf(f[3]) << 16);
-                lo.z = (uint32_t)f2bf(f[4]);
-            }
-            *(uint2*)(P + swz1(q, 0)) = make_uint2(lo.x, lo.y);
-            *(uint2*)(P + swz1(q, 1)) = make_uint2(lo.z, lo.w);
-            *(uint2*)(P + swz1(q, 2)) = make_uint2(hi.x, hi.y);
-            *(uint2*)(P + swz1(q, 3)) = make_uint2(hi.z, hi.w);
-        }
-        if (!RESIDENT) stage_weights(Wl, a.w[0], 9 * 32, false, tid, NT);
-        __syncthreads();
-        tile_layer1(P, Q, Wl, a.b[0], wave, lane, NW);
-        __syncthreads();
-        if (!RESIDENT) {
-            stage_weights(Wl, a.w[1], 9 * 32, true, tid, NT);
-            __syncthreads();
-        }
-        tile_layer32<32, false>(Q, 22, P, nullptr, 20, RESIDENT ? Wl + W_OFS1 : Wl, a.b[1], wave, lane, NW);
-        __syncthreads();
-        if (!RESIDENT) {
-            stage_weights(Wl, a.w[2], 9 * 32, true, tid, NT);
-            __syncthreads();
-        }
-        tile_layer32<32, false>(P, 20, Q, nullptr, 18, RESIDENT ? Wl + W_OFS2 : Wl, a.b[2], wave, lane, NW);
-        __syncthreads();
-        if (!RESIDENT) {
-            stage_weights(Wl, a.w[3], 9 * 16, true, tid, NT);
-            __syncthreads();
-        }
-        tile_layer32<16, true>(Q, 18, nullptr, OF, 16, RESIDENT ? Wl + W_OFS3 : Wl, a.b[3], wave, lane, NW);
-        __syncthreads();
-        for (int q = tid; q < 256; q += NT) {
-            const float r = OF[q * 3], g = OF[q * 3 + 1], b = OF[q * 3 + 2];
-            if (a.x) {
-                float* o = a.out + ((size_t)c * 256 + q) * 3;
-                o[0] = r;
-                o[1] = g;
-                o[2] = b;
-            } else {
-                V->staged[(size_t)lc * 256 + q] = rgb_word(r, g, b);
             }
         }
     }
@@ -745,7 +851,6 @@ struct svo_cnn {
     int2* origins = nullptr;
     int max_origins = 0;
     bool fused = true;     // per-tile fused inference kernel for the frame fill
-    int tile_mode = 0;     // fused kernel variant (see launch_tiles)
     bf16* xt = nullptr;    // explicit-mode tile inputs / outputs
     float* ot = nullptr;
     size_t cap_tiles = 0;
@@ -1172,23 +1277,15 @@ static TileArgs tile_args(svo_cnn* n)
     return a;
 }
 
-static unsigned tile_grid(int max_tiles, int cus, int per_cu)
+// grid > 0: that many workgroups, at most one per tile (they loop over the
+// tile list, so any count covers every tile); 0: two per CU
+static int launch_tiles(const TileArgs& a, int max_tiles, int cus, hipStream_t stream, int grid)
 {
-    return (unsigned)std::max(1, std::min(max_tiles, per_cu * cus));
-}
-
-// tile kernel variant: 0 = 4 waves, weights staged per layer (two workgroups
-// per CU); 1 = 8 waves, weights resident (one workgroup per CU)
-// (grid > 0: that many workgroups, at most one per tile; the workgroups loop
-// over the tile list, so any count covers every tile)
-static int launch_tiles(const TileArgs& a, int mode, int max_tiles, int cus, hipStream_t stream, int grid)
-{
-    const unsigned g1 = grid > 0 ? (unsigned)std::max(1, std::min(max_tiles, grid)) : tile_grid(max_tiles, cus, 1);
-    const unsigned g2 = grid > 0 ? (unsigned)std::max(1, std::min(max_tiles, grid)) : tile_grid(max_tiles, cus, 2);
-    if (mode == 1)
-        hipLaunchKernelGGL((k_cnn_tiles<8, true>), dim3(g1), dim3(512), 0, stream, a);
+    const unsigned g = (unsigned)std::max(1, std::min(max_tiles, grid > 0 ? grid : 2 * cus));
+    if (a.x)
+        hipLaunchKernelGGL(k_cnn_tiles<true>, dim3(g), dim3(256), 0, stream, a);
     else
-        hipLaunchKernelGGL((k_cnn_tiles<4, false>), dim3(g2), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL(k_cnn_tiles<false>, dim3(g), dim3(256), 0, stream, a);
     HIPCHECK(hipGetLastError());
     return SVO_OK;
 }
@@ -1220,7 +1317,7 @@ int cnn_fill_tiles(svo_cnn* n, svo_ctx* c, const svo_frame_params* p, const uint
     if (n->fused) {
         TileArgs a = tile_args(n);
         a.v = tile_view(c, p, tile_list, tile_count, max_tiles);
-        return launch_tiles(a, n->tile_mode, max_tiles, n->n_cu, stream, grid);
+        return launch_tiles(a, max_tiles, n->n_cu, stream, grid);
     }
     int rc = ensure_ws(n, (size_t)max_tiles * 576);
     if (rc) return rc;
@@ -1274,7 +1371,7 @@ int cnn_fill_tiles_batch(svo_cnn* n, svo_ctx* const* views, const svo_frame_para
     a.views = (const TileView*)d_tab;
     a.first = first;
     a.n_views = n_views;
-    return launch_tiles(a, n->tile_mode, max_all, n->n_cu, stream, 0);
+    return launch_tiles(a, max_all, n->n_cu, stream, 0);
 }
 
 // the staged colours of every view of a batch into their images (the table
@@ -1318,7 +1415,7 @@ extern "C" int svo_cnn_forward_tiles(svo_cnn* n, const uint16_t* x, int count, f
     a.x = n->xt;
     a.out = n->ot;
     a.n = count;
-    RCC(launch_tiles(a, n->tile_mode, count, n->n_cu, n->stream, 0));
+    RCC(launch_tiles(a, count, n->n_cu, n->stream, 0));
     HIPCHECK(hipMemcpyAsync(out, n->ot, (size_t)count * 256 * 3 * 4, hipMemcpyDeviceToHost, n->stream));
     HIPCHECK(hipStreamSynchronize(n->stream));
     return SVO_OK;
@@ -1329,6 +1426,5 @@ extern "C" int svo_cnn_set_fused(svo_cnn* n, int mode)
     if (!n) return svo_fail(SVO_ERR_ARG, "null network");
     if (mode < 0 || mode > 2) return svo_fail(SVO_ERR_ARG, "fused mode %d outside 0..2", mode);
     n->fused = mode != 0;
-    n->tile_mode = mode == 2 ? 1 : 0;
     return SVO_OK;
 }
