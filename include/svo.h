@@ -409,8 +409,8 @@ int svo_pretrace_stats(svo_ctx* ctx, uint64_t* rays, uint64_t* merged, uint32_t*
 /* Learned frames (svo_frame_warp_learned): the number of workgroups the
  * fused CNN tile kernel runs with while it shares the GPU with the ray
  * launch (0 = two per CU, its grid when it runs alone).  Fewer workgroups
- * take longer but leave the ray launch's SIMDs freer; the default is half
- * the CUs.  Batched learned frames and timing mode 1 use the full grid.
+ * take longer but leave the ray launch's SIMDs freer; the default is three
+ * quarters of the CUs.  Batched learned frames and timing mode 1 use the full grid.
  * No counterpart in the reference (it has no CNN); results do not depend
  * on it. */
 int svo_set_cnn_overlap(svo_ctx* ctx, int workgroups);

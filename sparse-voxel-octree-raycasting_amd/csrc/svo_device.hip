@@ -1340,7 +1340,12 @@ extern "C" int svo_create(svo_ctx** out, int device)
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
         c->n_cu = prop.multiProcessorCount;
-    c->cnn_overlap_wgs = std::max(1, c->n_cu / 2);
+    // The CNN tile kernel beside the ray launch: three quarters of the CUs.
+    // Learned frames back to back / each synced, us per frame: 1920x1024
+    // depth 11 at half 753 / 734, three quarters 636 / 663, all 626 / 666, two
+    // per CU 630 / 664; 1280x720 depth 10 710 / 780, 685 / 815, 700 / 832,
+    // 688 / 832; 640x480 314 / 445, 298 / 455, 295 / 470, 295 / 493.
+    c->cnn_overlap_wgs = std::max(1, c->n_cu * 3 / 4);
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess &&
               hipStreamCreateWithFlags(&c->cnn_stream, hipStreamNonBlocking) == hipSuccess;
     // the default pretrace's stream pool right behind the context's own two
