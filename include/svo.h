@@ -153,7 +153,7 @@ int svo_colorize(svo_ctx* ctx);
 /* ocl_copy_to_host (ocl.h:215-221): blocking read of `bytes` at byte_ofs. */
 int svo_read(svo_ctx* ctx, int buf, size_t byte_ofs, size_t bytes, void* dst);
 /* Non-blocking copy of the last frame's colorized image (SVO_BUF_IMAGE,
- * N uint32) into dst, on a copy stream of its own: the next call that
+ * N uint32) into dst, on a stream beside the frames': the next call that
  * rewrites the whole image (a frame, a batch frame or svo_colorize) renders
  * into a second image buffer meanwhile, so the copy overlaps it (the
  * reference uploads the image to a GL pixel buffer instead, raycast.h:
@@ -344,7 +344,9 @@ int svo_set_long_first(svo_ctx* ctx, int long_trips);
  * a frame is pretraced only while the warp frame before it is still on the
  * GPU (the caller issues frames ahead): a frame the GPU starts at once has
  * no earlier frame to overlap, and its own rays finish sooner without one.
- * Defaults: 3 sets, long_trips 1, 1 workgroup per CU, no split,
+ * Defaults: 3 sets (until the first svo_set_pretrace a frame whose
+ * predecessor was read with svo_read_image_async uses two of them, which
+ * leaves a hardware queue to the image copies), long_trips 1, 1 workgroup per CU, no split,
  * only_queued 1, predict 2, whole_trips 0, queue_skip 3.  A primary ray depends
  * only on the camera, the pixel and the octree (kernel.cl:594-694,
  * :846-942): results do not depend on these settings.  HIP maps streams onto

@@ -44,13 +44,15 @@ struct svo_ctx {
     uint32_t* d_ids = nullptr;
     uint32_t* d_image = nullptr;  // the frame's image: image_buf[0] or image_buf[1]
     // svo_read_image_async: a second image buffer, so the next frame renders
-    // into one while the other is copied to the host on copy_stream
+    // into one while the other is copied to the host (into pinned memory on
+    // cnn_stream, else on copy_stream)
     uint32_t* image_buf[2] = {nullptr, nullptr};
     hipStream_t copy_stream = nullptr;
     hipEvent_t image_ready = nullptr;
     hipEvent_t image_copied[2] = {nullptr, nullptr};
     bool image_copy_pending[2] = {false, false};
     bool image_flip = false;  // the next frame switches buffers
+    bool image_reads = false;  // the frame before this one was read with svo_read_image_async
     unsigned long long* d_keys = nullptr;
     uint32_t* d_snap = nullptr;
     int32_t* d_motion = nullptr;  // svo_fillhole_punch: motion x (N) then y (N)
@@ -102,6 +104,7 @@ struct svo_ctx {
     // earlier frames still run; the frame's own ray launch copies those of
     // its rays
     int pre_sets = 3;              // 0 = off
+    bool pre_auto = true;          // not set by the caller: 2 of the sets while images are read back
     uint32_t pre_trips = 1;
     int pre_wg = 1;                // workgroups per CU of the pretrace launch (0: wg_per_cu)
     int pre_split_trips = 0;       // blocks with a known ray this long go to the split waves (0: no split)

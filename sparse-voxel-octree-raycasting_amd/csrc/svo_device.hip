@@ -1067,6 +1067,47 @@ __global__ __launch_bounds__(256) void k_fill_color(View v, const View* views, c
     if (do_color) V.image[i] = colorize_word(w);
 }
 
+// ---------------------------------------------------------------- image to the host
+constexpr int kOutWgs = 8, kOutUnits = 4;  // working workgroups, 16-byte units per thread and round
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// Copy of an image to pinned host memory, n words; dst + head is 16-byte
+// aligned.  The host link takes 54 GB/s however many waves write to it, and
+// what else matters is the kernels that run meanwhile: stores that wait for
+// the link hold up every other miss of their L2.  So few waves write, all on
+// one XCD (workgroups go round the eight XCDs by index: only every eighth
+// works), past the caches.  7.9 MB, with a kernel beside it that streams
+// 71 MB in 11.1 us when alone: 8 working workgroups 147 us, the kernel beside
+// it 11.3; 4 145, 11.3; 2 243, 11.2; with cached stores 8 152, 12.0; a
+// workgroup per 16 KB on all XCDs 160, 121.6.  The runtime's copy engine
+// takes 151 us and leaves that kernel alone too, but a frame issued behind
+// such a copy starts late: full 1920x1024 frames with every image read back
+// 1010 us each against 770 (755 without reading), warp frames 512 against 440.
+__global__ __launch_bounds__(256) void k_image_out(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
+                                                   uint32_t n, uint32_t head)
+{
+    if (blockIdx.x % 8u) return;
+    const uint32_t wg = blockIdx.x / 8u;
+    // 16-byte units of dst; the `head` words before and the tail by word
+    const uint32_t n16 = (n - head) / 4u, end = head + n16 * 4u;
+    if (wg == 0 && threadIdx.x < head) dst[threadIdx.x] = src[threadIdx.x];
+    if (wg == 0 && threadIdx.x < n - end) dst[end + threadIdx.x] = src[end + threadIdx.x];
+    u32x4* const d = (u32x4*)(dst + head);
+    const uint32_t* const s = src + head;
+    for (uint32_t b = wg * 256u * kOutUnits; b < n16; b += kOutWgs * 256u * kOutUnits) {
+        u32x4 v[kOutUnits];
+#pragma unroll
+        for (int k = 0; k < kOutUnits; k++) {
+            const uint32_t i = min(b + k * 256u + threadIdx.x, n16 - 1u);
+            for (int j = 0; j < 4; j++) v[k][j] = s[4u * i + j];
+        }
+#pragma unroll
+        for (int k = 0; k < kOutUnits; k++) {
+            const uint32_t i = b + k * 256u + threadIdx.x;
+            if (i < n16) __builtin_nontemporal_store(v[k], d + i);
+        }
+    }
+}
+
 // ---------------------------------------------------------------- learned-fill gate
 // raycast_fine (kernel.cl:696-843, disabled in raycast.h:236): one ray per
 // 2x2 quad at (2 gx + add_x, 2 gy + add_y) over the rounded-up (res/4) grid
@@ -1269,9 +1310,20 @@ __global__ __launch_bounds__(256) void k_gate(View v, const View* views, int max
 
 static void free_pre(svo_ctx* c);
 
+// until every svo_read_image_async so far has its image
+static int wait_image_copies(svo_ctx* c)
+{
+    for (int s = 0; s < 2; s++) {
+        if (!c->image_copy_pending[s]) continue;
+        c->image_copy_pending[s] = false;
+        HIPCHECK(hipEventSynchronize(c->image_copied[s]));
+    }
+    return SVO_OK;
+}
+
 static int free_frame(svo_ctx* c)
 {
-    if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);  // no copy reads a freed image
+    (void)wait_image_copies(c);  // no copy reads a freed image
     if (c->d_image && c->d_image != c->image_buf[0] && c->d_image != c->image_buf[1])
         (void)hipFree(c->d_image);  // a resize that failed before recording it
     (void)hipFree(c->d_screen);
@@ -1548,6 +1600,7 @@ static int frame_end(svo_ctx* c)
 // that write part of the image or none keep the current buffer.
 static void take_image(svo_ctx* c)
 {
+    c->image_reads = c->image_flip;
     if (!c->image_flip || !c->image_buf[1]) return;
     c->image_flip = false;
     const int s = c->d_image == c->image_buf[1] ? 0 : 1;
@@ -2457,7 +2510,13 @@ static int pretrace_part(svo_ctx* c, const svo_frame_params* p, int s, int part,
 static int pretrace(svo_ctx* c, const svo_frame_params* p, int gate_max)
 {
     RC(ensure_pre(c));
-    const int s = (int)(c->pre_frames % (uint32_t)c->pre_sets);
+    // By default three sets, and two while the images are read back: then the
+    // copies need a hardware queue too (four, one of them the frames' own),
+    // and behind a pretrace's rays they would hold up the frame that waits for
+    // the image buffer.  Frames with every image read, three sets / two:
+    // 1920x1024 497 / 438 us, 1361x763 605 / 507, 1280x720 cave 298 / 269,
+    // learned 1920x1024 725 / 660; without reading 1361x763 340 / 460.
+    const int s = (int)(c->pre_frames % (uint32_t)(c->pre_auto && c->image_reads ? 2 : c->pre_sets));
     const uint32_t id = c->pre_frames + 1u;
     const bool pred = predict_ready(c, p);
     c->pre_early = pred && c->pre_whole_trips > 0;
@@ -2698,6 +2757,7 @@ extern "C" int svo_set_pretrace(svo_ctx* c, const svo_pretrace_config* cfg)
         free_pre(c);
         c->pre_sets = sets;
     }
+    c->pre_auto = false;
     c->pre_trips = (uint32_t)long_trips;
     c->pre_wg = wg_per_cu;
     c->pre_split_trips = cfg->split_trips;
@@ -3149,6 +3209,20 @@ extern "C" int svo_host_free(void* p)
     return SVO_OK;
 }
 
+// the device address of `bytes` of pinned host memory at p, or null when p is
+// anything else (or pinned for another device, or not word-aligned)
+static uint32_t* host_writable(const svo_ctx* c, void* p, size_t bytes)
+{
+    hipPointerAttribute_t a, z;
+    if (((uintptr_t)p & 3u) == 0 && hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeHost &&
+        a.device == c->device && a.devicePointer &&
+        hipPointerGetAttributes(&z, (char*)p + bytes - 1) == hipSuccess && z.type == hipMemoryTypeHost &&
+        (char*)z.devicePointer - (char*)a.devicePointer == (ptrdiff_t)bytes - 1)
+        return (uint32_t*)a.devicePointer;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 extern "C" int svo_read_image_async(svo_ctx* c, uint32_t* dst)
 {
     RC(need_frame(c));
@@ -3169,10 +3243,23 @@ extern "C" int svo_read_image_async(svo_ctx* c, uint32_t* dst)
         HIPCHECK(hipMemset(c->image_buf[1], 0, 4 * c->N));
     }
     const int s = c->d_image == c->image_buf[1] ? 1 : 0;
+    uint32_t* out = host_writable(c, dst, 4 * c->N);
+    // the kernel on the CNN's stream (idle in frames without a CNN, and a
+    // learned frame's CNN starts later than the copy of the one before ends):
+    // a stream of its own would be one more on the few hardware queues
+    hipStream_t st = out ? c->cnn_stream : c->copy_stream;
     HIPCHECK(hipEventRecord(c->image_ready, c->stream));
-    HIPCHECK(hipStreamWaitEvent(c->copy_stream, c->image_ready, 0));
-    HIPCHECK(hipMemcpyAsync(dst, c->d_image, 4 * c->N, hipMemcpyDeviceToHost, c->copy_stream));
-    HIPCHECK(hipEventRecord(c->image_copied[s], c->copy_stream));
+    HIPCHECK(hipStreamWaitEvent(st, c->image_ready, 0));
+    // a second read of the same image: its event stands for both
+    if (c->image_copy_pending[s]) HIPCHECK(hipStreamWaitEvent(st, c->image_copied[s], 0));
+    if (out) {
+        const uint32_t head = std::min((uint32_t)(-(uintptr_t)out & 15u) / 4u, (uint32_t)c->N);
+        hipLaunchKernelGGL(k_image_out, dim3(8 * kOutWgs), dim3(256), 0, st, c->d_image, out, (uint32_t)c->N, head);
+        HIPCHECK(hipGetLastError());
+    } else {
+        HIPCHECK(hipMemcpyAsync(dst, c->d_image, 4 * c->N, hipMemcpyDeviceToHost, st));
+    }
+    HIPCHECK(hipEventRecord(c->image_copied[s], st));
     c->image_copy_pending[s] = true;
     c->image_flip = true;
     return SVO_OK;
@@ -3196,10 +3283,7 @@ extern "C" int svo_sync(svo_ctx* c)
     if (!c) return svo_fail(SVO_ERR_ARG, "null context");
     HIPCHECK(hipSetDevice(c->device));
     HIPCHECK(hipStreamSynchronize(c->stream));
-    if (c->copy_stream) {
-        HIPCHECK(hipStreamSynchronize(c->copy_stream));
-        c->image_copy_pending[0] = c->image_copy_pending[1] = false;
-    }
+    RC(wait_image_copies(c));
     if (c->frame_timed) {
         c->frame_timed = false;
         int last = ST_N, first = -1;
