@@ -112,6 +112,12 @@ __global__ void k_level_start(const uint64_t* __restrict__ key, uint32_t L, int 
     if (starts(key, j, shift)) nstart[id] = j;
 }
 
+// nodes at each depth: the last entry of its inclusive scan
+__global__ void k_level_counts(int D, uint32_t L, Levels lv, uint32_t* __restrict__ count)
+{
+    if ((int)threadIdx.x < D) count[threadIdx.x] = lv.nid[threadIdx.x][L - 1];
+}
+
 // child (depth d+1, or leaf when d+1 == D) -> parent mask bit and creator index
 __global__ void k_level_link(const uint64_t* __restrict__ key, const uint32_t* __restrict__ leaf_first, uint32_t L,
                              int D, int d, Levels lv)
@@ -279,20 +285,38 @@ __global__ void k_emit_normal(int D, int d, Levels lv, const uint32_t* __restric
 
 inline unsigned blocks_for(size_t n) { return (unsigned)((n + 255) / 256); }
 
-// device allocations of one build, freed on every exit path
+// Device memory of one build, freed on every exit path.  Arrays are asked for
+// with want() and carved from one allocation per group: a build has four
+// groups (what is known with the voxel count, the leaves, the nodes, the
+// words), and an hipMalloc and hipFree pair takes 170 us or more: with one per
+// array (66) they were 11 of the 13 ms of a 4-million-voxel build.
 struct Pool {
+    struct Want {
+        void** p;
+        size_t ofs;
+    };
     std::vector<void*> ptrs;
+    std::vector<Want> wants;
+    size_t bytes = 0;
     ~Pool()
     {
         for (void* p : ptrs) (void)hipFree(p);
     }
     template <class T>
-    T* get(size_t count)
+    void want(T** p, size_t count)
     {
-        void* p = nullptr;
-        if (hipMalloc(&p, count * sizeof(T) + 16) != hipSuccess) return nullptr;
-        ptrs.push_back(p);
-        return (T*)p;
+        wants.push_back({(void**)p, bytes});
+        bytes += (count * sizeof(T) + 16 + 255) & ~(size_t)255;
+    }
+    bool carve()
+    {
+        char* base = nullptr;
+        if (hipMalloc((void**)&base, bytes) != hipSuccess) return false;
+        ptrs.push_back(base);
+        for (const Want& w : wants) *w.p = base + w.ofs;
+        wants.clear();
+        bytes = 0;
+        return true;
     }
 };
 
@@ -311,10 +335,10 @@ struct Stream {
         hipError_t e_ = (expr);                                                           \
         if (e_ != hipSuccess) return svo_fail(SVO_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
-#define BALLOC(ptr, T, count)                                                             \
+#define BCARVE()                                                                          \
     do {                                                                                  \
-        ptr = pool.get<T>(count);                                                         \
-        if (!ptr) return svo_fail(SVO_ERR_NOMEM, "octree build: %zu bytes", (size_t)(count) * sizeof(T)); \
+        const size_t bytes_ = pool.bytes;                                                 \
+        if (!pool.carve()) return svo_fail(SVO_ERR_NOMEM, "octree build: %zu bytes", bytes_); \
     } while (0)
 
 extern "C" int svo_build_octree_gpu(int device, const uint16_t* xyz, const uint32_t* rgba, size_t n, int depth,
@@ -343,23 +367,10 @@ extern "C" int svo_build_octree_gpu(int device, const uint16_t* xyz, const uint3
     Pool pool;
     const uint32_t N = (uint32_t)n;
 
-    uint16_t* d_xyz;
-    uint32_t *d_rgba, *d_idx, *d_idx2, *d_err, *d_flag;
-    uint64_t *d_key, *d_key2;
-    BALLOC(d_xyz, uint16_t, 3 * n);
-    BALLOC(d_rgba, uint32_t, n);
-    BALLOC(d_key, uint64_t, n);
-    BALLOC(d_key2, uint64_t, n);
-    BALLOC(d_idx, uint32_t, n);
-    BALLOC(d_idx2, uint32_t, n);
-    BALLOC(d_flag, uint32_t, n + 1);
-    BALLOC(d_err, uint32_t, 1);
-    BCHECK(hipMemcpyAsync(d_xyz, xyz, 6 * n, hipMemcpyHostToDevice, s));
-    BCHECK(hipMemcpyAsync(d_rgba, rgba, 4 * n, hipMemcpyHostToDevice, s));
-    BCHECK(hipMemsetAsync(d_err, 0, 4, s));
-    hipLaunchKernelGGL(k_morton, dim3(blocks_for(n)), dim3(256), 0, s, d_xyz, N, D, d_key, d_idx, d_err);
-    BCHECK(hipGetLastError());
-
+    uint16_t* d_xyz = nullptr;
+    uint32_t *d_rgba = nullptr, *d_idx = nullptr, *d_idx2 = nullptr, *d_err = nullptr, *d_flag = nullptr,
+             *d_lid = nullptr;
+    uint64_t *d_key = nullptr, *d_key2 = nullptr;
     // scratch for the library sort / scans, sized for the largest call
     size_t tmp_sort = 0, tmp_scan = 0;
     BCHECK(rocprim::radix_sort_pairs(nullptr, tmp_sort, d_key, d_key2, d_idx, d_idx2, N, 0u, (unsigned)(3 * D), s));
@@ -369,8 +380,24 @@ extern "C" int svo_build_octree_gpu(int device, const uint16_t* xyz, const uint3
     BCHECK(rocprim::exclusive_scan(nullptr, tmp_ex64, d_key, d_key2, (uint64_t)0, N + 1, rocprim::plus<uint64_t>(),
                                    s));
     size_t tmp_bytes = std::max(std::max(tmp_sort, tmp_scan), std::max(tmp_ex32, tmp_ex64));
-    void* d_tmp;
-    BALLOC(d_tmp, char, tmp_bytes);
+    char* d_tmp;
+    pool.want(&d_xyz, 3 * n);
+    pool.want(&d_rgba, n);
+    pool.want(&d_key, n);
+    pool.want(&d_key2, n);
+    pool.want(&d_idx, n);
+    pool.want(&d_idx2, n);
+    pool.want(&d_flag, n + 1);
+    pool.want(&d_lid, n);
+    pool.want(&d_err, 1 + kMaxLevels);
+    pool.want(&d_tmp, tmp_bytes);
+    BCARVE();
+    BCHECK(hipMemcpyAsync(d_xyz, xyz, 6 * n, hipMemcpyHostToDevice, s));
+    BCHECK(hipMemcpyAsync(d_rgba, rgba, 4 * n, hipMemcpyHostToDevice, s));
+    BCHECK(hipMemsetAsync(d_err, 0, 4, s));
+    hipLaunchKernelGGL(k_morton, dim3(blocks_for(n)), dim3(256), 0, s, d_xyz, N, D, d_key, d_idx, d_err);
+    BCHECK(hipGetLastError());
+
     BCHECK(rocprim::radix_sort_pairs(d_tmp, tmp_sort, d_key, d_key2, d_idx, d_idx2, N, 0u, (unsigned)(3 * D), s));
     uint32_t herr = 0;
     BCHECK(hipMemcpyAsync(&herr, d_err, 4, hipMemcpyDeviceToHost, s));
@@ -378,8 +405,6 @@ extern "C" int svo_build_octree_gpu(int device, const uint16_t* xyz, const uint3
     if (herr) return svo_fail(SVO_ERR_ARG, "a voxel lies outside 2^%d", D);
 
     // unique leaves
-    uint32_t* d_lid;
-    BALLOC(d_lid, uint32_t, n);
     hipLaunchKernelGGL(k_heads, dim3(blocks_for(n)), dim3(256), 0, s, d_key2, N, d_flag);
     BCHECK(hipGetLastError());
     size_t tb = tmp_bytes;
@@ -387,57 +412,68 @@ extern "C" int svo_build_octree_gpu(int device, const uint16_t* xyz, const uint3
     uint32_t L = 0;
     BCHECK(hipMemcpyAsync(&L, d_lid + (N - 1), 4, hipMemcpyDeviceToHost, s));
     BCHECK(hipStreamSynchronize(s));
-    uint64_t* d_lkey;
-    uint32_t *d_lfirst, *d_lcolor;
-    BALLOC(d_lkey, uint64_t, L);
-    BALLOC(d_lfirst, uint32_t, L);
-    BALLOC(d_lcolor, uint32_t, L);
+    Levels lv;
+    memset(&lv, 0, sizeof(lv));
+    uint64_t *d_lkey, *d_W, *d_sW;
+    uint32_t *d_lfirst, *d_lcolor, *d_C, *d_sC;
+    pool.want(&d_lkey, L);
+    pool.want(&d_lfirst, L);
+    pool.want(&d_lcolor, L);
+    for (int d = 0; d < D; d++) pool.want(&lv.nid[d], L);
+    pool.want(&d_W, (size_t)L + 1);
+    pool.want(&d_C, (size_t)L + 1);
+    pool.want(&d_sW, (size_t)L + 1);
+    pool.want(&d_sC, (size_t)L + 1);
+    BCARVE();
     hipLaunchKernelGGL(k_leaves, dim3(blocks_for(n)), dim3(256), 0, s, d_key2, d_idx2, d_rgba, d_lid, N, d_lkey,
                        d_lfirst, d_lcolor);
     BCHECK(hipGetLastError());
 
-    // nodes per depth
-    Levels lv;
-    memset(&lv, 0, sizeof(lv));
+    // nodes per depth; the counts of all depths in one read
     for (int d = 0; d < D; d++) {
-        const int shift = 3 * (D - d);
-        BALLOC(lv.nid[d], uint32_t, L);
-        hipLaunchKernelGGL(k_level_flags, dim3(blocks_for(L)), dim3(256), 0, s, d_lkey, L, shift, d_flag);
+        hipLaunchKernelGGL(k_level_flags, dim3(blocks_for(L)), dim3(256), 0, s, d_lkey, L, 3 * (D - d), d_flag);
         BCHECK(hipGetLastError());
         tb = tmp_bytes;
         BCHECK(rocprim::inclusive_scan(d_tmp, tb, d_flag, lv.nid[d], L, rocprim::plus<uint32_t>(), s));
-        uint32_t cnt = 0;
-        BCHECK(hipMemcpyAsync(&cnt, lv.nid[d] + (L - 1), 4, hipMemcpyDeviceToHost, s));
-        BCHECK(hipStreamSynchronize(s));
-        lv.count[d] = cnt;
-        BALLOC(lv.nstart[d], uint32_t, cnt);
-        BALLOC(lv.mask[d], uint32_t, cnt);
-        BALLOC(lv.first[d], uint32_t, cnt);
-        BALLOC(lv.ofs[d], uint32_t, cnt);
-        BCHECK(hipMemsetAsync(lv.mask[d], 0, 4 * (size_t)cnt, s));
-        BCHECK(hipMemsetAsync(lv.first[d], 0xff, 4 * (size_t)cnt, s));
-        BCHECK(hipMemsetAsync(lv.ofs[d], 0, 4 * (size_t)cnt, s));
-        hipLaunchKernelGGL(k_level_start, dim3(blocks_for(L)), dim3(256), 0, s, d_lkey, L, shift, lv.nid[d],
-                           lv.nstart[d]);
+    }
+    hipLaunchKernelGGL(k_level_counts, dim3(1), dim3(64), 0, s, D, L, lv, d_err + 1);
+    BCHECK(hipGetLastError());
+    BCHECK(hipMemcpyAsync(lv.count, d_err + 1, 4 * D, hipMemcpyDeviceToHost, s));
+    BCHECK(hipStreamSynchronize(s));
+    size_t nodes = 0;
+    for (int d = 0; d < D; d++) nodes += lv.count[d];
+    const uint32_t nblk = lv.count[D - 6];
+    uint32_t *d_nbytes, *d_nstart, *d_mask, *d_ofs, *d_first;
+    uint64_t *d_bsize, *d_bsize64, *d_bpos;
+    pool.want(&d_mask, nodes);  // masks, offsets and byte counts start at zero: one fill
+    pool.want(&d_ofs, nodes);
+    pool.want(&d_nbytes, lv.count[D - 2]);
+    const size_t zeroed = pool.bytes;
+    pool.want(&d_first, nodes);
+    pool.want(&d_nstart, nodes);
+    pool.want(&d_bsize, nblk);
+    pool.want(&d_bsize64, nblk);
+    pool.want(&d_bpos, nblk);
+    BCARVE();
+    BCHECK(hipMemsetAsync(d_mask, 0, zeroed, s));
+    BCHECK(hipMemsetAsync(d_first, 0xff, 4 * nodes, s));
+    for (size_t d = 0, o = 0; (int)d < D; o += lv.count[d++]) {
+        lv.nstart[d] = d_nstart + o;
+        lv.mask[d] = d_mask + o;
+        lv.first[d] = d_first + o;
+        lv.ofs[d] = d_ofs + o;
+        hipLaunchKernelGGL(k_level_start, dim3(blocks_for(L)), dim3(256), 0, s, d_lkey, L, 3 * (D - (int)d),
+                           lv.nid[d], lv.nstart[d]);
         BCHECK(hipGetLastError());
     }
     for (int d = D - 1; d >= 0; d--) {
         hipLaunchKernelGGL(k_level_link, dim3(blocks_for(L)), dim3(256), 0, s, d_lkey, d_lfirst, L, D, d, lv);
         BCHECK(hipGetLastError());
     }
-    uint32_t* d_nbytes;
-    BALLOC(d_nbytes, uint32_t, lv.count[D - 2]);
-    BCHECK(hipMemsetAsync(d_nbytes, 0, 4 * (size_t)lv.count[D - 2], s));
     hipLaunchKernelGGL(k_bytecount, dim3(blocks_for(L)), dim3(256), 0, s, d_lcolor, L, lv.nid[D - 2], d_nbytes);
     BCHECK(hipGetLastError());
 
     // post-order offsets
-    uint64_t *d_W, *d_sW;
-    uint32_t *d_C, *d_sC;
-    BALLOC(d_W, uint64_t, (size_t)L + 1);
-    BALLOC(d_C, uint32_t, (size_t)L + 1);
-    BALLOC(d_sW, uint64_t, (size_t)L + 1);
-    BALLOC(d_sC, uint32_t, (size_t)L + 1);
     hipLaunchKernelGGL(k_chain, dim3(blocks_for((size_t)L + 1)), dim3(256), 0, s, d_lkey, L, D, lv, d_nbytes, d_W,
                        d_C);
     BCHECK(hipGetLastError());
@@ -447,11 +483,6 @@ extern "C" int svo_build_octree_gpu(int device, const uint16_t* xyz, const uint3
     BCHECK(rocprim::exclusive_scan(d_tmp, tb, d_C, d_sC, 0u, L + 1, rocprim::plus<uint32_t>(), s));
     hipLaunchKernelGGL(k_offsets, dim3(blocks_for(L)), dim3(256), 0, s, d_lkey, L, D, lv, d_nbytes, d_sW, d_sC);
     BCHECK(hipGetLastError());
-    const uint32_t nblk = lv.count[D - 6];
-    uint64_t *d_bsize, *d_bsize64, *d_bpos;
-    BALLOC(d_bsize, uint64_t, nblk);
-    BALLOC(d_bsize64, uint64_t, nblk);
-    BALLOC(d_bpos, uint64_t, nblk);
     hipLaunchKernelGGL(k_block_size, dim3(blocks_for(nblk)), dim3(256), 0, s, L, D, lv, d_sW, d_bsize, d_bsize64);
     BCHECK(hipGetLastError());
     tb = tmp_bytes;
@@ -468,7 +499,8 @@ extern "C" int svo_build_octree_gpu(int device, const uint16_t* xyz, const uint3
     if ((uint64_t)n_normal * 10u > kNormalWords) return svo_fail(SVO_ERR_ARG, "normal region exceeds 2^21 words");
 
     uint32_t* d_out;
-    BALLOC(d_out, uint32_t, total);
+    pool.want(&d_out, total);
+    BCARVE();
     BCHECK(hipMemsetAsync(d_out, 0, 4 * total, s));
     for (int d = D - 6; d <= D - 3; d++) {
         hipLaunchKernelGGL(k_emit_compact, dim3(blocks_for(lv.count[d])), dim3(256), 0, s, D, d, lv, d_rgba, d_bpos,

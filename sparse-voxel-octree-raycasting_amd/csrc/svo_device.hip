@@ -1492,7 +1492,9 @@ extern "C" int svo_upload_octree(svo_ctx* c, const uint32_t* words, size_t n_wor
     (void)hipFree(c->d_oct);
     c->d_oct = nullptr;
     HIPCHECK(hipMalloc(&c->d_oct, (n_words + kOctPad) * 4));
-    HIPCHECK(hipMemcpy(c->d_oct, dev.data(), n_words * 4, hipMemcpyHostToDevice));
+    // the array as it is, then its renumbered first words over it
+    HIPCHECK(hipMemcpy(c->d_oct, words, n_words * 4, hipMemcpyHostToDevice));
+    HIPCHECK(hipMemcpy(c->d_oct, dev.data(), (size_t)normal_words * 4, hipMemcpyHostToDevice));
     HIPCHECK(hipMemset(c->d_oct + n_words, 0, kOctPad * 4));
     c->n_words = n_words;
     c->root = new_root;

@@ -12,8 +12,9 @@ int svo_fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)
 int svo_host_threads();
 
 #include <vector>
-// Validated device copy of a compact word array with the normal region in
-// breadth-first order; *normal_words = size of the renumbered region;
+// Validates a compact word array and renumbers its normal region in
+// breadth-first order: `out` = the region's new words, *normal_words of them,
+// which replace the array's first ones (the words after them stay);
 // *one_depth = no normal record is reached at two depths (true of every
 // built octree), so a node's depth tells what kind of node it is.
 int svo_device_layout(const uint32_t* words, size_t n_words, uint32_t root, int depth,

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import weakref
 
 import numpy as np
 
@@ -187,9 +188,13 @@ class PretraceConfig(C.Structure):
 
 
 def _take_u32(p, n):
-    a = np.ctypeslib.as_array(p, (n,)).copy()
-    _f["free"](C.cast(p, _vp))
-    return a
+    """The n words at p as an array that frees them with its last view."""
+    if n == 0:
+        _f["free"](C.cast(p, _vp))
+        return np.empty(0, np.uint32)
+    buf = (C.c_uint32 * n).from_address(C.addressof(p.contents))
+    weakref.finalize(buf, _f["free"], C.cast(p, _vp)).atexit = False
+    return np.frombuffer(buf, np.uint32)
 
 
 # ------------------------------------------------------------------ host helpers
