@@ -38,11 +38,26 @@ __device__ __forceinline__ bf16 f2bf(float f)
 }
 __device__ __forceinline__ float bf2f(bf16 h) { return __uint_as_float((uint32_t)h << 16); }
 constexpr uint32_t HOLE_WORD = 0xffffff00u;
+// The four layers' channels, and the flat parameter vector: per layer W
+// [9][cout][cin] then b [cout].  kWofs counts weights only (the bf16 copies).
+constexpr int kCin[4] = {16, 32, 32, 32}, kCout[4] = {32, 32, 32, 16};
+constexpr int kWofs[5] = {0, 4608, 13824, 23040, 27648};
+constexpr int kPofs[5] = {0, 4640, 13888, 23136, 27760};
+constexpr int kParams = kPofs[4];
+// the layer that holds index i of one of these tables
+__device__ __forceinline__ int layer_of(const int (&ofs)[5], int i)
+{
+    return (i >= ofs[1]) + (i >= ofs[2]) + (i >= ofs[3]);
+}
 constexpr int TILE = 8;          // output tile edge per wave
 constexpr int HALO = TILE + 2;   // input tile edge
 
 // MODE 0: + bias, ReLU, bf16 out.  MODE 1: + bias, fp32 out (last layer).
 // MODE 2: no bias, multiplied by (mask_src > 0), bf16 out (backward data).
+// At training sizes a SIMD has one wave, so latency bounds it: the halo's
+// loads go out together, the masks of the backward before the products, and
+// the taps are unrolled so that the weights are read ahead.  16 crops of
+// 64x64, 32 -> 32 channels: forward 10.8 -> 7.8 us, backward 16.5 -> 8.8.
 // Work items (crop, 8x8 tile) are taken grid-stride; the crop count is B, or
 // min(*bcount, B) when bcount is given (batches sized on the device).
 template <int CIN, int COUT, int MODE>
@@ -61,21 +76,38 @@ __global__ __launch_bounds__(64) void k_conv(const bf16* __restrict__ X, const b
     const int y0 = (t / tiles_x) * TILE, x0 = (t % tiles_x) * TILE;
     __syncthreads();  // previous item's LDS reads are done
     // stage the (TILE+2)^2 x CIN input halo, zero outside the crop
-    for (int i = lane; i < HALO * HALO * (CIN / 4); i += 64) {
-        const int pix = i / (CIN / 4), c4 = (i % (CIN / 4)) * 4;
+    constexpr int UNITS = HALO * HALO * (CIN / 4), LOADS = (UNITS + 63) / 64;
+    uint2 v[LOADS];
+#pragma unroll
+    for (int k = 0; k < LOADS; k++) {
+        const int i = lane + 64 * k, pix = i / (CIN / 4), c4 = (i % (CIN / 4)) * 4;
         const int yy = y0 + pix / HALO - 1, xx = x0 + pix % HALO - 1;
-        uint2 v = make_uint2(0u, 0u);
-        if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-            v = *(const uint2*)(X + (((size_t)b * H + yy) * W + xx) * CIN + c4);
-        *(uint2*)(xs + pix * CS + c4) = v;
+        v[k] = make_uint2(0u, 0u);
+        if (i < UNITS && yy >= 0 && yy < H && xx >= 0 && xx < W)
+            v[k] = *(const uint2*)(X + (((size_t)b * H + yy) * W + xx) * CIN + c4);
     }
+#pragma unroll
+    for (int k = 0; k < LOADS; k++) {
+        const int i = lane + 64 * k;
+        if (i < UNITS) *(uint2*)(xs + i / (CIN / 4) * CS + (i % (CIN / 4)) * 4) = v[k];
+    }
+    constexpr int NT = COUT / 16;
+    const int row = lane & 15, kq = (lane >> 4) * 4;
+    // backward: the ReLU masks are read ahead of the products
+    bf16 keep[4][NT][4];
+    if (MODE == 2)
+        for (int m = 0; m < 4; m++)
+            for (int n = 0; n < NT; n++)
+                for (int i = 0; i < 4; i++) {
+                    const int p = m * 16 + kq + i, py = p / TILE, px = p % TILE;
+                    keep[m][n][i] = mask_src[(((size_t)b * H + y0 + py) * W + x0 + px) * COUT + n * 16 + row];
+                }
     __syncthreads();
 
-    constexpr int NT = COUT / 16;
     f4v acc[4][NT];
     for (int m = 0; m < 4; m++)
         for (int n = 0; n < NT; n++) acc[m][n] = f4v{0.f, 0.f, 0.f, 0.f};
-    const int row = lane & 15, kq = (lane >> 4) * 4;
+#pragma unroll
     for (int tap = 0; tap < 9; tap++) {
         const int dy = tap / 3, dx = tap % 3;
         for (int kc = 0; kc < CIN / 16; kc++) {
@@ -106,70 +138,120 @@ __global__ __launch_bounds__(64) void k_conv(const bf16* __restrict__ X, const b
                     ((float*)Yout)[o] = v + bias[co];
                 } else {
                     // ReLU derivative: the forward output (>= 0) is positive
-                    ((bf16*)Yout)[o] = mask_src[o] != 0 ? f2bf(v) : (bf16)0;
+                    ((bf16*)Yout)[o] = keep[m][n][i] != 0 ? f2bf(v) : (bf16)0;
                 }
             }
         }
     }
 }
 
-// dW partial of crop b: sum over the crop's pixels p of dZ[p][co] X[p + tap
-// - 1][ci].  grid = (crops, 9 taps), DW_SLICES waves per workgroup: wave s
-// loops over pixel slice s (a multiple of 16 pixels), K = 16 pixels per MFMA
-// (A = dZ^T: co x pixels, B = shifted X: pixels x ci); the waves' sums are
-// added in slice order through LDS and written to part[b][tap][co][ci];
-// k_sum_parts adds the crops' partials in crop order, so the gradient does
-// not depend on scheduling.
+// The gradients of layers lo .. lo + gridDim.z - 1 in one launch (dz of every
+// layer is kept): a layer by itself has 9 workgroups per crop, which leaves
+// most CUs idle at the usual 16 to 32 crops.
+struct GradArgs {
+    const bf16* x[4];   // a layer's input
+    const bf16* dz[4];  // the gradient of its output before the ReLU
+    float* part_w;      // per layer [B][9][cout][cin], from layer lo on
+    float* part_b;      // per layer [db blocks][32]
+    float* grads;       // flat, as the parameters
+    int B, H, W, lo, db_blocks;
+};
+
+// dW partials of crop b: sum over the crop's pixels p of dZ[p][co] X[p + tap
+// - 1][ci].  grid = (crops, 3 tap rows, layers), DW_SLICES waves per
+// workgroup: wave s loops over pixel slice s (a multiple of 16 pixels), K = 16
+// pixels per MFMA (A = dZ^T: co x pixels, B = shifted X: pixels x ci); the
+// waves' sums are added in slice order through LDS and written to
+// part[b][tap][co][ci]; k_sum_grads adds the crops' partials in crop order, so
+// the gradient does not depend on scheduling.
+// Both operands are read transposed, two bytes at a time, so the loads and
+// their addresses bound it.  A row's three taps share them: 8 for dZ and, as
+// the taps' four pixels overlap, 12 for X instead of 48 (all 32 channels).
+// 16 crops of 64x64, all layers: 98 us with a launch per layer and a tap per
+// workgroup, 70 so in one launch, 20 with the three taps.
 constexpr int DW_SLICES = 16;
 template <int CIN, int COUT>
-__global__ __launch_bounds__(64 * DW_SLICES) void k_conv_dw(const bf16* __restrict__ X, const bf16* __restrict__ dZ,
-                                                            float* __restrict__ part, int H, int W)
+__device__ __forceinline__ void conv_dw(const bf16* __restrict__ X, const bf16* __restrict__ dZ,
+                                        float* __restrict__ part, int H, int W, float* s_acc)
 {
-    __shared__ float s_acc[DW_SLICES][COUT * CIN];
-    const int b = blockIdx.x, tap = blockIdx.y, sl = threadIdx.x >> 6;
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
+    const int b = blockIdx.x, dy = (int)blockIdx.y - 1, sl = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63, row = lane & 15, kq = (lane >> 4) * 4;
     constexpr int MT = COUT / 16, NT = CIN / 16;
-    f4v acc[MT][NT];
-    for (int m = 0; m < MT; m++)
-        for (int n = 0; n < NT; n++) acc[m][n] = f4v{0.f, 0.f, 0.f, 0.f};
+    f4v acc[3][MT][NT];
+    for (int t = 0; t < 3; t++)
+        for (int m = 0; m < MT; m++)
+            for (int n = 0; n < NT; n++) acc[t][m][n] = f4v{0.f, 0.f, 0.f, 0.f};
     const int npix = H * W;  // a multiple of 16
     const int len = (npix / 16 + DW_SLICES - 1) / DW_SLICES * 16;
     const int kb = min(npix, sl * len), ke = min(npix, kb + len);
-    const bf16* dz = dZ + (size_t)b * npix * COUT;
-    const bf16* xb = X + (size_t)b * npix * CIN;
-    for (int k0 = kb; k0 < ke; k0 += 16) {
-        s4v afr[MT], bfr[NT];
-        for (int m = 0; m < MT; m++) {
-            short tmp[4];
-            for (int j = 0; j < 4; j++) tmp[j] = (short)dz[(size_t)(k0 + kq + j) * COUT + m * 16 + row];
-            afr[m] = s4v{tmp[0], tmp[1], tmp[2], tmp[3]};
-        }
-        for (int n = 0; n < NT; n++) {
-            short tmp[4];
-            for (int j = 0; j < 4; j++) {
-                const int p = k0 + kq + j, y = p / W + dy, x = p % W + dx;
-                tmp[j] = (y >= 0 && y < H && x >= 0 && x < W) ? (short)xb[((size_t)y * W + x) * CIN + n * 16 + row] : 0;
+    const bf16* dz = dZ + (size_t)b * npix * COUT + row;
+    const bf16* xb = X + (size_t)b * npix * CIN + row;
+    constexpr int U = 2;  // steps whose loads are issued together
+    for (int k0 = kb; k0 < ke; k0 += 16 * U) {
+        s4v afr[U][MT], bfr[U][3][NT];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            // past the slice: the last step's addresses again, and zeros
+            const bool in = k0 + 16 * u < ke;
+            const int p = min(k0 + 16 * u, ke - 16) + kq;
+            const bf16* za = dz + p * COUT;
+            for (int m = 0; m < MT; m++) {
+                s4v v;
+                for (int j = 0; j < 4; j++) v[j] = (short)za[j * COUT + m * 16];
+                afr[u][m] = in ? v : s4v{0, 0, 0, 0};
             }
-            bfr[n] = s4v{tmp[0], tmp[1], tmp[2], tmp[3]};
+            // p is a multiple of 4 and W of 8: the four pixels share a row,
+            // and only the pixel before and the one after can be outside it
+            const int y = p / W + dy, x = p % W;
+            const bool in_y = in && y >= 0 && y < H, in_l = in_y && x > 0, in_r = in_y && x + 4 < W;
+            const bf16* xa = xb + (min(max(y, 0), H - 1) * W + x) * CIN;
+            const bf16* xl = xa - (x > 0 ? CIN : 0);
+            const bf16* xr = xa + (x + 4 < W ? 4 : 3) * CIN;
+            for (int n = 0; n < NT; n++) {
+                short v[6];
+                v[0] = (short)xl[n * 16];
+                for (int j = 0; j < 4; j++) v[j + 1] = (short)xa[j * CIN + n * 16];
+                v[5] = (short)xr[n * 16];
+                v[0] = in_l ? v[0] : (short)0;
+                for (int j = 1; j < 5; j++) v[j] = in_y ? v[j] : (short)0;
+                v[5] = in_r ? v[5] : (short)0;
+                for (int t = 0; t < 3; t++) bfr[u][t][n] = s4v{v[t], v[t + 1], v[t + 2], v[t + 3]};
+            }
         }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            for (int t = 0; t < 3; t++)
+                for (int m = 0; m < MT; m++)
+                    for (int n = 0; n < NT; n++)
+                        acc[t][m][n] =
+                            __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(afr[u][m], bfr[u][t][n], acc[t][m][n], 0, 0, 0);
+    }
+    for (int t = 0; t < 3; t++) {
+        if (t) __syncthreads();  // the tap before has been read
         for (int m = 0; m < MT; m++)
             for (int n = 0; n < NT; n++)
-                acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(afr[m], bfr[n], acc[m][n], 0, 0, 0);
+                for (int i = 0; i < 4; i++) {
+                    const int co = m * 16 + kq + i, ci = n * 16 + row;
+                    s_acc[sl * COUT * CIN + co * CIN + ci] = acc[t][m][n][i];
+                }
+        __syncthreads();
+        float* dw = part + ((size_t)b * 9 + blockIdx.y * 3 + t) * COUT * CIN;
+        for (int e = threadIdx.x; e < COUT * CIN; e += 64 * DW_SLICES) {
+            float v = 0.f;
+            for (int k = 0; k < DW_SLICES; k++) v += s_acc[k * COUT * CIN + e];
+            dw[e] = v;
+        }
     }
-    for (int m = 0; m < MT; m++)
-        for (int n = 0; n < NT; n++)
-            for (int i = 0; i < 4; i++) {
-                const int co = m * 16 + kq + i, ci = n * 16 + row;
-                s_acc[sl][co * CIN + ci] = acc[m][n][i];
-            }
-    __syncthreads();
-    float* dw = part + ((size_t)b * 9 + tap) * COUT * CIN;
-    for (int e = threadIdx.x; e < COUT * CIN; e += 64 * DW_SLICES) {
-        float t = 0.f;
-        for (int k = 0; k < DW_SLICES; k++) t += s_acc[k][e];
-        dw[e] = t;
-    }
+}
+
+__global__ __launch_bounds__(64 * DW_SLICES) void k_conv_dw(GradArgs a)
+{
+    __shared__ float s_acc[DW_SLICES * 32 * 32];
+    const int l = a.lo + (int)blockIdx.z;
+    float* part = a.part_w + (size_t)a.B * (kWofs[l] - kWofs[a.lo]);
+    if (l == 0) conv_dw<16, 32>(a.x[0], a.dz[0], part, a.H, a.W, s_acc);
+    else if (l == 3) conv_dw<32, 16>(a.x[3], a.dz[3], part, a.H, a.W, s_acc);
+    else conv_dw<32, 32>(a.x[l], a.dz[l], part, a.H, a.W, s_acc);
 }
 
 // db partial of block b: part[b][co] = sum over its DB_PIXELS pixels of
@@ -177,12 +259,12 @@ __global__ __launch_bounds__(64 * DW_SLICES) void k_conv_dw(const bf16* __restri
 // channel in order)
 constexpr int DB_PIXELS = 256;
 template <int COUT>
-__global__ __launch_bounds__(256) void k_conv_db(const bf16* __restrict__ dZ, float* __restrict__ part, int npix)
+__device__ __forceinline__ void conv_db(const bf16* __restrict__ dZ, float* __restrict__ part, int npix, float* s_sum)
 {
-    __shared__ float s_sum[256];
     const int co = threadIdx.x % COUT, lane_p = threadIdx.x / COUT;
     const int p0 = blockIdx.x * DB_PIXELS, p1 = min(p0 + DB_PIXELS, npix);
     float s = 0.f;
+#pragma unroll 8
     for (int p = p0 + lane_p; p < p1; p += 256 / COUT) s += bf2f(dZ[(size_t)p * COUT + co]);
     s_sum[threadIdx.x] = s;
     __syncthreads();
@@ -192,35 +274,59 @@ __global__ __launch_bounds__(256) void k_conv_db(const bf16* __restrict__ dZ, fl
         part[(size_t)blockIdx.x * COUT + threadIdx.x] = t;
     }
 }
-
-// out[e] for many partials and few elements (one workgroup per element):
-// thread t sums part[t], part[t + 256], ... in order, then a fixed pairwise
-// tree over the 256 threads
-__global__ __launch_bounds__(256) void k_sum_parts_tree(const float* __restrict__ part, int n_parts, int n,
-                                                        float* __restrict__ out)
+__global__ __launch_bounds__(256) void k_conv_db(GradArgs a)
 {
+    __shared__ float s_sum[256];
+    const int l = a.lo + (int)blockIdx.y;
+    float* part = a.part_b + (size_t)a.db_blocks * 32 * blockIdx.y;
+    const int npix = a.B * a.H * a.W;
+    if (l == 3) conv_db<16>(a.dz[3], part, npix, s_sum);
+    else conv_db<32>(a.dz[l], part, npix, s_sum);
+}
+
+// The partials added up, layers lo .. hi - 1.  The first workgroups take 256
+// weights each (a layer's are a multiple of 256): one thread per weight adds
+// the crops in order.  The others take one bias each: thread t adds partials
+// t, t + 256, ... in order, then a fixed pairwise tree over the 256 threads.
+__global__ __launch_bounds__(256) void k_sum_grads(GradArgs a, int hi)
+{
+    const int wblocks = (kWofs[hi] - kWofs[a.lo]) / 256;
+    const int t = threadIdx.x;
+    if ((int)blockIdx.x < wblocks) {
+        const int i = kWofs[a.lo] + (int)blockIdx.x * 256 + t;
+        const int l = layer_of(kWofs, i), n = kWofs[l + 1] - kWofs[l], e = i - kWofs[l];
+        const float* part = a.part_w + (size_t)a.B * (kWofs[l] - kWofs[a.lo]) + e;
+        float s = 0.f;
+#pragma unroll 8
+        for (int p = 0; p < a.B; p++) s += part[(size_t)p * n];
+        a.grads[kPofs[l] + e] = s;
+        return;
+    }
     __shared__ float s[256];
-    const int e = blockIdx.x, t = threadIdx.x;
+    const int bi = (int)blockIdx.x - wblocks, l = a.lo + bi / 32, e = bi % 32;  // (layer 3 has 16 biases)
+    const int n = kCout[l];
+    const float* part = a.part_b + (size_t)a.db_blocks * 32 * (l - a.lo) + e;
     float v = 0.f;
-    for (int p = t; p < n_parts; p += 256) v += part[(size_t)p * n + e];
+    for (int p = t; p < a.db_blocks; p += 256) v += part[(size_t)p * n];
     s[t] = v;
     __syncthreads();
     for (int h = 128; h > 0; h >>= 1) {
         if (t < h) s[t] += s[t + h];
         __syncthreads();
     }
-    if (t == 0) out[e] = s[0];
+    if (t == 0) a.grads[kPofs[l + 1] - n + e] = s[0];
 }
 
-// out[e] = sum over p = 0 .. n_parts-1, in order, of part[p][e]
-__global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ part, int n_parts, int n,
-                                                   float* __restrict__ out)
+// *sum += v of every thread of a workgroup of 256, one atomic (16 ns each on
+// the same word: one per thread or per wave took 16 us at 65,536 pixels)
+__device__ __forceinline__ void add_once(float v, float* sum)
 {
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= n) return;
-    float s = 0.f;
-    for (int p = 0; p < n_parts; p++) s += part[(size_t)p * n + e];
-    out[e] = s;
+    __shared__ float s[4];
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    if (__lane_id() == 0) s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = (s[0] + s[1]) + (s[2] + s[3]);
+    if (threadIdx.x == 0 && v != 0.f) atomicAdd(sum, v);
 }
 
 // masked MSE on RGB: loss += sum mask*(pred-t)^2 / (3*count); dZ = d loss/d pred
@@ -228,20 +334,22 @@ __global__ __launch_bounds__(256) void k_loss(const float* __restrict__ pred, co
                                               const float* __restrict__ mask, bf16* dZ, float* loss, int npix,
                                               const float* __restrict__ mask_count)
 {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= npix) return;
     const float inv_count = *mask_count > 0.f ? 1.f / (3.f * *mask_count) : 0.f;
     float l = 0.f;
-    for (int c = 0; c < 16; c++) {
-        float g = 0.f;
-        if (c < 3) {
+    for (int p = blockIdx.x * 256 + threadIdx.x; p < npix; p += gridDim.x * 256) {
+        uint32_t g[3];
+        float lp = 0.f;
+        for (int c = 0; c < 3; c++) {
             const float d = pred[(size_t)p * 16 + c] - target[(size_t)p * 3 + c];
-            l += mask[p] * d * d;
-            g = 2.f * mask[p] * d * inv_count;
+            lp += mask[p] * d * d;
+            g[c] = f2bf(2.f * mask[p] * d * inv_count);
         }
-        dZ[(size_t)p * 16 + c] = f2bf(g);
+        l += lp * inv_count;
+        uint4* z = (uint4*)(dZ + (size_t)p * 16);
+        z[0] = make_uint4(g[0] | (g[1] << 16), g[2], 0u, 0u);
+        z[1] = make_uint4(0u, 0u, 0u, 0u);
     }
-    if (l != 0.f) atomicAdd(loss, l * inv_count);
+    add_once(l, loss);
 }
 
 // Input features of crop c (origin from `origins`, or tile list -> tile*16-4):
@@ -320,8 +428,10 @@ __global__ __launch_bounds__(256) void k_features(FeatArgs a)
                 tb = (float)(px & 255u) * (1.f / 255.f);
             }
         }
-        bf16* xo = a.x + i * 16;
-        for (int k = 0; k < 16; k++) xo[k] = k < 5 ? f2bf(f[k]) : (bf16)0;
+        uint4* xo = (uint4*)(a.x + i * 16);
+        xo[0] = make_uint4(f2bf(f[0]) | ((uint32_t)f2bf(f[1]) << 16), f2bf(f[2]) | ((uint32_t)f2bf(f[3]) << 16),
+                           f2bf(f[4]), 0u);
+        xo[1] = make_uint4(0u, 0u, 0u, 0u);
         if (a.target) {
             a.target[i * 3 + 0] = tr;
             a.target[i * 3 + 1] = tg;
@@ -330,7 +440,8 @@ __global__ __launch_bounds__(256) void k_features(FeatArgs a)
             cnt += m;
         }
     }
-    if (a.target && cnt != 0.f) atomicAdd(a.mask_count, cnt);
+    if (!a.target) return;
+    add_once(cnt, a.mask_count);
 }
 
 __device__ __forceinline__ uint32_t rgb_word(float r, float g, float b)
@@ -786,64 +897,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-// W'[t][ci][co] = W[8-t][co][ci] (backward-data weights), bf16
-__global__ void k_flip(const float* __restrict__ W, bf16* Wf, int cin, int cout)
+// All parameters at once: with kStep an Adam step first (FP32 master weights;
+// m, v moments, bias-corrected), then the weights' bf16 copies, forward
+// [9][cout][cin] and for the backward data W'[t][ci][co] = W[8-t][co][ci].
+// (16 launches of 2.5 us each and the gaps between them before.)
+template <bool kStep>
+__global__ __launch_bounds__(256) void k_params(float* __restrict__ w, const float* __restrict__ g,
+                                                float* __restrict__ m, float* __restrict__ v,
+                                                bf16* __restrict__ wbf, bf16* __restrict__ wflip, float lr, float b1,
+                                                float b2, float c1, float c2, float eps)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= 9 * cin * cout) return;
-    const int t = i / (cin * cout), r = i % (cin * cout), ci = r / cout, co = r % cout;
-    Wf[i] = f2bf(W[((size_t)(8 - t) * cout + co) * cin + ci]);
-}
-
-__global__ void k_to_bf16(const float* __restrict__ a, bf16* b, int n)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) b[i] = f2bf(a[i]);
-}
-
-// Adam (FP32 master weights): m, v moments, bias-corrected step
-__global__ void k_adam(float* w, const float* g, float* m, float* v, int n, float lr, float b1, float b2,
-                       float c1, float c2, float eps)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    if (i >= kParams) return;
+    float x = w[i];
+    if (kStep) {
+        const float gi = g[i];
+        const float mi = b1 * m[i] + (1.f - b1) * gi;
+        const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
+        m[i] = mi;
+        v[i] = vi;
+        x -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+        w[i] = x;
+    }
+    const int l = layer_of(kPofs, i), e = i - kPofs[l], cin = kCin[l], cout = kCout[l], per = cin * cout;
+    if (e >= 9 * per) return;  // a bias
+    const int t = e / per, co = e % per / cin, ci = e % cin;
+    const bf16 h = f2bf(x);
+    wbf[kWofs[l] + e] = h;
+    wflip[kWofs[l] + ((8 - t) * cin + ci) * cout + co] = h;
 }
 
 }  // namespace
 
 // ====================================================================== host
 struct CnnLayer {
-    int cin, cout;
-    size_t nw;          // 9*cin*cout
-    float* w = nullptr; // fp32 master [9][cout][cin]
-    float* b = nullptr; // fp32 [cout]
-    float* gw = nullptr;
-    float* gb = nullptr;
-    float *mw = nullptr, *vw = nullptr, *mb = nullptr, *vb = nullptr;
-    bf16* wbf = nullptr;   // forward weights
-    bf16* wflip = nullptr; // backward-data weights [9][cin][cout]
+    float* w;     // fp32 master [9][cout][cin]
+    float* b;     // fp32 [cout]
+    bf16* wbf;    // forward weights
+    bf16* wflip;  // backward-data weights [9][cin][cout]
 };
 
 struct svo_cnn {
     int device = 0;
     int n_cu = 256;        // compute units of the device (tile kernel grid)
     hipStream_t stream = nullptr;
-    CnnLayer L[4];
+    CnnLayer L[4] = {};  // into params, wbf, wflip
+    float *params = nullptr, *grads = nullptr, *m = nullptr, *v = nullptr;  // flat, kParams each
+    bf16 *wbf = nullptr, *wflip = nullptr;
+    float* h_grads = nullptr;  // pinned: kParams gradients and the loss
     int step = 0;
     // activation workspace for the current batch size
     size_t cap_pix = 0;
     bf16* x0 = nullptr;    // [pix][16]
     bf16* y[3] = {};       // [pix][32]
     float* out = nullptr;  // [pix][16]
-    bf16* dz16 = nullptr;  // [pix][16]
-    bf16* dz32a = nullptr; // [pix][32]
-    bf16* dz32b = nullptr; // [pix][32]
+    bf16* dz[4] = {};      // [pix][32], the last layer's [pix][16]
     float* target = nullptr;
     float* mask = nullptr;
     float* loss = nullptr;
@@ -854,7 +962,7 @@ struct svo_cnn {
     bf16* xt = nullptr;    // explicit-mode tile inputs / outputs
     float* ot = nullptr;
     size_t cap_tiles = 0;
-    float* part = nullptr;  // gradient partials (per crop and tap, or per block)
+    float* part = nullptr;  // gradient partials: per crop and tap, then per block
     size_t cap_part = 0;
 };
 
@@ -871,22 +979,18 @@ struct svo_cnn {
             return svo_fail(SVO_ERR_HIP, "%s failed: %s", #expr, hipGetErrorString(_e)); \
     } while (0)
 
-static const int kCin[4] = {16, 32, 32, 32}, kCout[4] = {32, 32, 32, 16};
-
 static void free_ws(svo_cnn* n)
 {
     (void)hipFree(n->x0);
     for (auto& p : n->y) (void)hipFree(p);
     (void)hipFree(n->out);
-    (void)hipFree(n->dz16);
-    (void)hipFree(n->dz32a);
-    (void)hipFree(n->dz32b);
+    for (auto& p : n->dz) (void)hipFree(p);
     (void)hipFree(n->target);
     (void)hipFree(n->mask);
     n->x0 = nullptr;
     for (auto& p : n->y) p = nullptr;
     n->out = nullptr;
-    n->dz16 = n->dz32a = n->dz32b = nullptr;
+    for (auto& p : n->dz) p = nullptr;
     n->target = n->mask = nullptr;
     n->cap_pix = 0;
 }
@@ -897,9 +1001,9 @@ static int ensure_ws(svo_cnn* n, size_t pix)
     free_ws(n);
     bool ok = hipMalloc(&n->x0, pix * 16 * 2) == hipSuccess && hipMalloc(&n->y[0], pix * 32 * 2) == hipSuccess &&
               hipMalloc(&n->y[1], pix * 32 * 2) == hipSuccess && hipMalloc(&n->y[2], pix * 32 * 2) == hipSuccess &&
-              hipMalloc(&n->out, pix * 16 * 4) == hipSuccess && hipMalloc(&n->dz16, pix * 16 * 2) == hipSuccess &&
-              hipMalloc(&n->dz32a, pix * 32 * 2) == hipSuccess && hipMalloc(&n->dz32b, pix * 32 * 2) == hipSuccess &&
+              hipMalloc(&n->out, pix * 16 * 4) == hipSuccess &&
               hipMalloc(&n->target, pix * 3 * 4) == hipSuccess && hipMalloc(&n->mask, pix * 4) == hipSuccess;
+    for (int l = 0; l < 4; l++) ok = ok && hipMalloc(&n->dz[l], pix * kCout[l] * 2) == hipSuccess;
     if (!ok) {
         free_ws(n);
         return svo_fail(SVO_ERR_NOMEM, "CNN workspace for %zu pixels", pix);
@@ -912,10 +1016,8 @@ static unsigned nb(size_t n) { return (unsigned)((n + 255) / 256); }
 
 static int refresh_bf16(svo_cnn* n)
 {
-    for (auto& l : n->L) {
-        hipLaunchKernelGGL(k_to_bf16, dim3(nb(l.nw)), dim3(256), 0, n->stream, l.w, l.wbf, (int)l.nw);
-        hipLaunchKernelGGL(k_flip, dim3(nb(l.nw)), dim3(256), 0, n->stream, l.w, l.wflip, l.cin, l.cout);
-    }
+    hipLaunchKernelGGL(k_params<false>, dim3(nb(kParams)), dim3(256), 0, n->stream, n->params, (const float*)nullptr,
+                       (float*)nullptr, (float*)nullptr, n->wbf, n->wflip, 0.f, 0.f, 0.f, 1.f, 1.f, 0.f);
     HIPCHECK(hipGetLastError());
     return SVO_OK;
 }
@@ -926,11 +1028,10 @@ extern "C" int svo_cnn_destroy(svo_cnn* n)
     (void)hipSetDevice(n->device);
     (void)hipStreamSynchronize(n->stream);
     free_ws(n);
-    for (auto& l : n->L) {
-        for (float* p : {l.w, l.b, l.gw, l.gb, l.mw, l.vw, l.mb, l.vb}) (void)hipFree(p);
-        (void)hipFree(l.wbf);
-        (void)hipFree(l.wflip);
-    }
+    for (float* p : {n->params, n->grads, n->m, n->v}) (void)hipFree(p);
+    (void)hipFree(n->wbf);
+    (void)hipFree(n->wflip);
+    (void)hipHostFree(n->h_grads);
     (void)hipFree(n->loss);
     (void)hipFree(n->mask_count);
     (void)hipFree(n->part);
@@ -944,9 +1045,7 @@ extern "C" int svo_cnn_destroy(svo_cnn* n)
 
 extern "C" size_t svo_cnn_param_count(void)
 {
-    size_t s = 0;
-    for (int i = 0; i < 4; i++) s += 9 * (size_t)kCin[i] * kCout[i] + kCout[i];
-    return s;
+    return kParams;
 }
 
 extern "C" int svo_cnn_create(svo_cnn** out, int device, uint64_t seed)
@@ -974,32 +1073,28 @@ extern "C" int svo_cnn_create(svo_cnn** out, int device, uint64_t seed)
         return ((z ^ (z >> 31)) >> 11) * (1.0 / 9007199254740992.0);
     };
     const int real_in[4] = {5, 32, 32, 32}, real_out[4] = {32, 32, 32, 3};
+    std::vector<float> w(kParams, 0.f);
     for (int li = 0; li < 4; li++) {
-        CnnLayer& l = n->L[li];
-        l.cin = kCin[li];
-        l.cout = kCout[li];
-        l.nw = 9 * (size_t)l.cin * l.cout;
-        std::vector<float> w(l.nw, 0.f), b(l.cout, 0.f);
         const double sd = sqrt(2.0 / (9.0 * real_in[li])) * (li == 3 ? 0.5 : 1.0);
         for (int t = 0; t < 9; t++)
             for (int co = 0; co < real_out[li]; co++)
                 for (int ci = 0; ci < real_in[li]; ci++) {
                     double u1 = std::max(next(), 1e-12), u2 = next();
-                    w[((size_t)t * l.cout + co) * l.cin + ci] = (float)(sd * sqrt(-2 * log(u1)) * cos(6.283185307179586 * u2));
+                    w[kPofs[li] + (t * kCout[li] + co) * kCin[li] + ci] = (float)(sd * sqrt(-2 * log(u1)) * cos(6.283185307179586 * u2));
                 }
-        bool ok = true;
-        for (float** p : {&l.w, &l.gw, &l.mw, &l.vw}) ok = ok && hipMalloc(p, l.nw * 4) == hipSuccess;
-        for (float** p : {&l.b, &l.gb, &l.mb, &l.vb}) ok = ok && hipMalloc(p, l.cout * 4) == hipSuccess;
-        ok = ok && hipMalloc(&l.wbf, l.nw * 2) == hipSuccess && hipMalloc(&l.wflip, l.nw * 2) == hipSuccess;
-        if (!ok) {
-            svo_cnn_destroy(n);
-            return svo_fail(SVO_ERR_NOMEM, "CNN weights");
-        }
-        (void)hipMemcpy(l.w, w.data(), l.nw * 4, hipMemcpyHostToDevice);
-        (void)hipMemcpy(l.b, b.data(), l.cout * 4, hipMemcpyHostToDevice);
-        for (float* p : {l.mw, l.vw}) (void)hipMemset(p, 0, l.nw * 4);
-        for (float* p : {l.mb, l.vb}) (void)hipMemset(p, 0, l.cout * 4);
     }
+    bool ok = true;
+    for (float** p : {&n->params, &n->grads, &n->m, &n->v}) ok = ok && hipMalloc(p, kParams * 4) == hipSuccess;
+    for (bf16** p : {&n->wbf, &n->wflip}) ok = ok && hipMalloc(p, kWofs[4] * 2) == hipSuccess;
+    ok = ok && hipHostMalloc((void**)&n->h_grads, (kParams + 1) * 4, hipHostMallocDefault) == hipSuccess;
+    if (!ok) {
+        svo_cnn_destroy(n);
+        return svo_fail(SVO_ERR_NOMEM, "CNN weights");
+    }
+    (void)hipMemcpy(n->params, w.data(), kParams * 4, hipMemcpyHostToDevice);
+    for (float* p : {n->m, n->v}) (void)hipMemset(p, 0, kParams * 4);
+    for (int l = 0; l < 4; l++)
+        n->L[l] = {n->params + kPofs[l], n->params + kPofs[l + 1] - kCout[l], n->wbf + kWofs[l], n->wflip + kWofs[l]};
     int rc = refresh_bf16(n);
     if (rc) {
         svo_cnn_destroy(n);
@@ -1015,12 +1110,7 @@ extern "C" int svo_cnn_get_params(svo_cnn* n, float* dst, size_t count)
 {
     if (!n || !dst || count != svo_cnn_param_count()) return svo_fail(SVO_ERR_ARG, "need %zu floats", svo_cnn_param_count());
     HIPCHECK(hipStreamSynchronize(n->stream));
-    for (auto& l : n->L) {
-        HIPCHECK(hipMemcpy(dst, l.w, l.nw * 4, hipMemcpyDeviceToHost));
-        dst += l.nw;
-        HIPCHECK(hipMemcpy(dst, l.b, l.cout * 4, hipMemcpyDeviceToHost));
-        dst += l.cout;
-    }
+    HIPCHECK(hipMemcpy(dst, n->params, kParams * 4, hipMemcpyDeviceToHost));
     return SVO_OK;
 }
 
@@ -1028,12 +1118,7 @@ extern "C" int svo_cnn_set_params(svo_cnn* n, const float* src, size_t count)
 {
     if (!n || !src || count != svo_cnn_param_count()) return svo_fail(SVO_ERR_ARG, "need %zu floats", svo_cnn_param_count());
     HIPCHECK(hipStreamSynchronize(n->stream));
-    for (auto& l : n->L) {
-        HIPCHECK(hipMemcpy(l.w, src, l.nw * 4, hipMemcpyHostToDevice));
-        src += l.nw;
-        HIPCHECK(hipMemcpy(l.b, src, l.cout * 4, hipMemcpyHostToDevice));
-        src += l.cout;
-    }
+    HIPCHECK(hipMemcpy(n->params, src, kParams * 4, hipMemcpyHostToDevice));
     return refresh_bf16(n);
 }
 
@@ -1054,14 +1139,20 @@ int cnn_forward_dev(svo_cnn* n, int B, int H, int W, const uint32_t* bcount = nu
     return SVO_OK;
 }
 
-// backward from n->out vs n->target/n->mask; gradients into L[].gw/gb
+// Partials of all layers' weights at most: beyond it (more than 2,427 crops)
+// the gradients are made layer by layer through one layer's partials.
+constexpr size_t kPartBytes = (size_t)1 << 28;
+
+// backward from n->out vs n->target/n->mask; gradients into n->grads
 // (per-crop and per-block partials added in a fixed order)
 int cnn_backward_dev(svo_cnn* n, int B, int H, int W)
 {
     const size_t pix = (size_t)B * H * W;
     const unsigned g = conv_grid(B, H, W);
     const unsigned gdb = (unsigned)((pix + DB_PIXELS - 1) / DB_PIXELS);
-    const size_t need = std::max((size_t)B * 9 * 32 * 32, (size_t)gdb * 32);
+    const int together = (size_t)B * kWofs[4] * 4 <= kPartBytes ? 4 : 1;  // layers per launch
+    const size_t need_w = (size_t)B * (together == 4 ? kWofs[4] : 9 * 32 * 32);
+    const size_t need = need_w + (size_t)gdb * 32 * together;
     if (need > n->cap_part) {
         (void)hipFree(n->part);
         n->part = nullptr;
@@ -1070,41 +1161,24 @@ int cnn_backward_dev(svo_cnn* n, int B, int H, int W)
         n->cap_part = need;
     }
     HIPCHECK(hipMemsetAsync(n->loss, 0, 4, n->stream));
-    hipLaunchKernelGGL(k_loss, dim3(nb(pix)), dim3(256), 0, n->stream, n->out, n->target, n->mask, n->dz16, n->loss,
-                       (int)pix, n->mask_count);
-    // weight and bias gradients of layer l from its input X and output gradient dZ
-    auto dwdb = [&](int l, const bf16* X, const bf16* dZ) {
-        CnnLayer& L = n->L[l];
-        const dim3 gdw((unsigned)B, 9), bdw(64 * DW_SLICES);
-        if (l == 3)
-            hipLaunchKernelGGL((k_conv_dw<32, 16>), gdw, bdw, 0, n->stream, X, dZ, n->part, H, W);
-        else if (l == 0)
-            hipLaunchKernelGGL((k_conv_dw<16, 32>), gdw, bdw, 0, n->stream, X, dZ, n->part, H, W);
-        else
-            hipLaunchKernelGGL((k_conv_dw<32, 32>), gdw, bdw, 0, n->stream, X, dZ, n->part, H, W);
-        hipLaunchKernelGGL(k_sum_parts, dim3(nb(L.nw)), dim3(256), 0, n->stream, (const float*)n->part, B,
-                           (int)L.nw, L.gw);
-        if (l == 3)
-            hipLaunchKernelGGL((k_conv_db<16>), dim3(gdb), dim3(256), 0, n->stream, dZ, n->part, (int)pix);
-        else
-            hipLaunchKernelGGL((k_conv_db<32>), dim3(gdb), dim3(256), 0, n->stream, dZ, n->part, (int)pix);
-        hipLaunchKernelGGL(k_sum_parts_tree, dim3((unsigned)L.cout), dim3(256), 0, n->stream, (const float*)n->part,
-                           (int)gdb, L.cout, L.gb);
-    };
-    // layer 4 (32 -> 16)
-    dwdb(3, n->y[2], n->dz16);
-    hipLaunchKernelGGL((k_conv<16, 32, 2>), dim3(g), dim3(64), 0, n->stream, n->dz16, n->L[3].wflip,
-                       (const float*)nullptr, n->y[2], (void*)n->dz32a, H, W, B, (const uint32_t*)nullptr);
-    // layer 3
-    dwdb(2, n->y[1], n->dz32a);
-    hipLaunchKernelGGL((k_conv<32, 32, 2>), dim3(g), dim3(64), 0, n->stream, n->dz32a, n->L[2].wflip,
-                       (const float*)nullptr, n->y[1], (void*)n->dz32b, H, W, B, (const uint32_t*)nullptr);
-    // layer 2
-    dwdb(1, n->y[0], n->dz32b);
-    hipLaunchKernelGGL((k_conv<32, 32, 2>), dim3(g), dim3(64), 0, n->stream, n->dz32b, n->L[1].wflip,
-                       (const float*)nullptr, n->y[0], (void*)n->dz32a, H, W, B, (const uint32_t*)nullptr);
-    // layer 1 (16 -> 32)
-    dwdb(0, n->x0, n->dz32a);
+    hipLaunchKernelGGL(k_loss, dim3(std::min(nb(pix / 4), 1024u)), dim3(256), 0, n->stream, n->out, n->target,
+                       n->mask, n->dz[3], n->loss, (int)pix, n->mask_count);
+    hipLaunchKernelGGL((k_conv<16, 32, 2>), dim3(g), dim3(64), 0, n->stream, n->dz[3], n->L[3].wflip,
+                       (const float*)nullptr, n->y[2], (void*)n->dz[2], H, W, B, (const uint32_t*)nullptr);
+    hipLaunchKernelGGL((k_conv<32, 32, 2>), dim3(g), dim3(64), 0, n->stream, n->dz[2], n->L[2].wflip,
+                       (const float*)nullptr, n->y[1], (void*)n->dz[1], H, W, B, (const uint32_t*)nullptr);
+    hipLaunchKernelGGL((k_conv<32, 32, 2>), dim3(g), dim3(64), 0, n->stream, n->dz[1], n->L[1].wflip,
+                       (const float*)nullptr, n->y[0], (void*)n->dz[0], H, W, B, (const uint32_t*)nullptr);
+    GradArgs a{{n->x0, n->y[0], n->y[1], n->y[2]}, {n->dz[0], n->dz[1], n->dz[2], n->dz[3]},
+               n->part, n->part + need_w, n->grads, B, H, W, 0, (int)gdb};
+    for (; a.lo < 4; a.lo += together) {
+        const int hi = a.lo + together;
+        const int biases = 32 * (together - 1) + kCout[hi - 1];
+        hipLaunchKernelGGL(k_conv_dw, dim3((unsigned)B, 3, (unsigned)together), dim3(64 * DW_SLICES), 0, n->stream, a);
+        hipLaunchKernelGGL(k_conv_db, dim3(gdb, (unsigned)together), dim3(256), 0, n->stream, a);
+        hipLaunchKernelGGL(k_sum_grads, dim3((unsigned)((kWofs[hi] - kWofs[a.lo]) / 256 + biases)), dim3(256), 0,
+                           n->stream, a, hi);
+    }
     HIPCHECK(hipGetLastError());
     return SVO_OK;
 }
@@ -1114,14 +1188,10 @@ int cnn_adam_dev(svo_cnn* n, float lr)
     n->step++;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.f - powf(b1, (float)n->step), c2 = 1.f - powf(b2, (float)n->step);
-    for (auto& l : n->L) {
-        hipLaunchKernelGGL(k_adam, dim3(nb(l.nw)), dim3(256), 0, n->stream, l.w, l.gw, l.mw, l.vw, (int)l.nw, lr, b1,
-                           b2, c1, c2, 1e-8f);
-        hipLaunchKernelGGL(k_adam, dim3(nb(l.cout)), dim3(256), 0, n->stream, l.b, l.gb, l.mb, l.vb, l.cout, lr, b1,
-                           b2, c1, c2, 1e-8f);
-    }
+    hipLaunchKernelGGL(k_params<true>, dim3(nb(kParams)), dim3(256), 0, n->stream, n->params, (const float*)n->grads,
+                       n->m, n->v, n->wbf, n->wflip, lr, b1, b2, c1, c2, 1e-8f);
     HIPCHECK(hipGetLastError());
-    return refresh_bf16(n);
+    return SVO_OK;
 }
 
 static int check_shape(int B, int H, int W)
@@ -1165,18 +1235,16 @@ extern "C" int svo_cnn_gradients(svo_cnn* n, const uint16_t* x, const float* tar
     HIPCHECK(hipMemcpyAsync(n->x0, x, pix * 16 * 2, hipMemcpyHostToDevice, n->stream));
     HIPCHECK(hipMemcpyAsync(n->target, target, pix * 3 * 4, hipMemcpyHostToDevice, n->stream));
     HIPCHECK(hipMemcpyAsync(n->mask, mask, pix * 4, hipMemcpyHostToDevice, n->stream));
-    float cnt = 0.f;
+    if ((rc = cnn_forward_dev(n, B, H, W))) return rc;
+    float cnt = 0.f;  // while the forward runs
     for (size_t i = 0; i < pix; i++) cnt += mask[i];
     HIPCHECK(hipMemcpyAsync(n->mask_count, &cnt, 4, hipMemcpyHostToDevice, n->stream));
-    if ((rc = cnn_forward_dev(n, B, H, W)) || (rc = cnn_backward_dev(n, B, H, W))) return rc;
+    if ((rc = cnn_backward_dev(n, B, H, W))) return rc;
+    HIPCHECK(hipMemcpyAsync(n->h_grads, n->grads, kParams * 4, hipMemcpyDeviceToHost, n->stream));
+    HIPCHECK(hipMemcpyAsync(n->h_grads + kParams, n->loss, 4, hipMemcpyDeviceToHost, n->stream));
     HIPCHECK(hipStreamSynchronize(n->stream));
-    for (auto& l : n->L) {
-        HIPCHECK(hipMemcpy(grads, l.gw, l.nw * 4, hipMemcpyDeviceToHost));
-        grads += l.nw;
-        HIPCHECK(hipMemcpy(grads, l.gb, l.cout * 4, hipMemcpyDeviceToHost));
-        grads += l.cout;
-    }
-    HIPCHECK(hipMemcpy(loss, n->loss, 4, hipMemcpyDeviceToHost));
+    memcpy(grads, n->h_grads, kParams * 4);
+    *loss = n->h_grads[kParams];
     return SVO_OK;
 }
 
@@ -1246,7 +1314,8 @@ extern "C" int svo_cnn_train_step(svo_cnn* n, svo_ctx* warp, svo_ctx* full, cons
     a.target = n->target;
     a.mask = n->mask;
     a.mask_count = n->mask_count;
-    hipLaunchKernelGGL(k_features, dim3(1024), dim3(256), 0, n->stream, a);
+    const size_t pix = (size_t)n_crops * crop * crop;
+    hipLaunchKernelGGL(k_features, dim3(std::min(nb(pix / 2), 1024u)), dim3(256), 0, n->stream, a);
     HIPCHECK(hipGetLastError());
     if ((rc = cnn_forward_dev(n, n_crops, crop, crop)) || (rc = cnn_backward_dev(n, n_crops, crop, crop)) ||
         (rc = cnn_adam_dev(n, lr)))
