@@ -756,30 +756,40 @@ __global__ __launch_bounds__(RAY_BLOCK) void k_rays(RayArgs a)
 // The copy half of a frame's rays with a pretrace: every ray of the view
 // whose pixel carries the frame's stamp takes the pretraced word and
 // position (what finish_ray would write; the other rays were traced by the
-// launch before).  One thread per ray; merged rays counted into *merged.
+// launch before); merged rays counted into *merged.  The host does not know
+// the lists' lengths: a thread per possible ray was 20 us at 1920x1024, nearly
+// all of it workgroups without a ray; kMergeWgs workgroups that go round the
+// actual rays take 12 at 1280x720 (24 before).  1280x720 cave clip with
+// read-back 2157 -> 1885 us, 1920x1024 flight 3540 -> 3460; 256 and 1,024
+// workgroups the same.
+constexpr unsigned kMergeWgs = 512;
 __global__ __launch_bounds__(256) void k_pre_merge(View v, unsigned long long* merged)
 {
     const View& V = v;
-    const uint32_t k = blockIdx.x * 256u + threadIdx.x;
-    int x = 0, y = 0;
-    uint32_t blk;
-    bool took = false;
-    if (k < view_rays(V) && ray_pixel(V, k, x, y, blk)) {
+    const uint32_t rays = view_rays(V);
+    uint32_t n = 0;
+    for (uint32_t k = blockIdx.x * 256u + threadIdx.x; k < rays; k += gridDim.x * 256u) {
+        int x = 0, y = 0;
+        uint32_t blk;
+        if (!ray_pixel(V, k, x, y, blk)) continue;
         const uint32_t pix = (uint32_t)(y * V.res_x + x);
-        if (V.pre_stamp[pix] == V.pre_id) {
-            const uint32_t word = V.pre_word[pix];
-            const float4 q = V.pre_xyz[pix];
-            V.screen[pix] = word;
-            float* c = (float*)V.coords + 4u * pix;
-            c[0] = q.x;
-            c[1] = q.y;
-            c[2] = q.z;
-            if (V.ray_image) V.ray_image[pix] = colorize_word(word);
-            took = true;
-        }
+        if (V.pre_stamp[pix] != V.pre_id) continue;
+        const uint32_t word = V.pre_word[pix];
+        const float4 q = V.pre_xyz[pix];
+        V.screen[pix] = word;
+        float* c = (float*)V.coords + 4u * pix;
+        c[0] = q.x;
+        c[1] = q.y;
+        c[2] = q.z;
+        if (V.ray_image) V.ray_image[pix] = colorize_word(word);
+        n++;
     }
-    const unsigned long long b = __ballot(took);
-    if (__lane_id() == 0 && b) atomicAdd(merged, (unsigned long long)__popcll(b));
+    __shared__ uint32_t s_n;
+    if (threadIdx.x == 0) s_n = 0u;
+    __syncthreads();
+    if (n) atomicAdd(&s_n, n);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_n) atomicAdd(merged, (unsigned long long)s_n);
 }
 
 // ---------------------------------------------------------------- warp
@@ -1868,9 +1878,7 @@ static int frame_rays(svo_ctx* c, View v)
     HIPCHECK(hipStreamWaitEvent(c->stream, c->ev_pre[2 * s + 1], 0));
     if (c->pre_early) HIPCHECK(hipStreamWaitEvent(c->stream, c->ev_pre[2 * s], 0));
     v.pre_mode = 2;
-    // one thread per possible ray: both lists hold at most N pixels each
-    const size_t n = (v.list ? c->N : 0) + (v.list2 ? c->N : 0) + v.n_rect;
-    hipLaunchKernelGGL(k_pre_merge, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, v,
+    hipLaunchKernelGGL(k_pre_merge, dim3(kMergeWgs), dim3(256), 0, c->stream, v,
                        (unsigned long long*)(c->d_queue + 12));
     HIPCHECK(hipGetLastError());
     return SVO_OK;
