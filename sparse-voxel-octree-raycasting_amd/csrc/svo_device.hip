@@ -144,7 +144,7 @@ struct View {
     const uint32_t* rect_skip;   // per 8x8 block: nonzero = raycast from the list instead, or null
     uint32_t* block_long;        // per 8x8 block: set to 1 by a ray of >= long_trips trips, or null
     uint32_t long_trips;
-    // learned frames: destination of the CNN input copy (plane 0 after the gate)
+    // learned frames: destination of the CNN input copy (plane 0 at the gate)
     uint32_t* cnn_words;
     float4* cnn_coords;
     // learned-fill gate of this view: counters, CNN tile list, gate pixel list
@@ -960,16 +960,23 @@ __global__ __launch_bounds__(1024) void k_sumids(View v, const View* views, uint
     }
 }
 
-// first ray of each batched view (after their compaction), one thread
-__global__ void k_view_first(const View* views, int n, uint32_t* first, uint32_t* zero)
+// first ray of each batched view (after their compaction), one wave
+__global__ __launch_bounds__(64) void k_view_first(const View* views, int n, uint32_t* first, uint32_t* zero)
 {
-    if (zero) *zero = 0u;  // the ray-queue counter of the launch that follows
+    const int lane = threadIdx.x;
+    if (zero && lane == 0) *zero = 0u;  // the ray-queue counter of the launch that follows
     uint32_t acc = 0;
-    for (int i = 0; i < n; i++) {
-        first[i] = acc;
-        acc += view_rays(views[i]);
+    for (int b = 0; b < n; b += 64) {
+        const uint32_t rays = b + lane < n ? view_rays(views[b + lane]) : 0u;
+        uint32_t incl = rays;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t t = __shfl_up(incl, d);
+            if (lane >= d) incl += t;
+        }
+        if (b + lane < n) first[b + lane] = acc + incl - rays;
+        acc += __shfl(incl, 63);
     }
-    first[n] = acc;
+    if (lane == 0) first[n] = acc;
 }
 
 // ---------------------------------------------------------------- copy / filter / colorize
@@ -981,17 +988,6 @@ __global__ __launch_bounds__(256) void k_copy_plane(View v, const View* views, u
     const size_t d = (size_t)dst_plane * V.N + i;
     V.screen[d] = V.screen[i];
     V.coords[d] = V.coords[i];
-}
-
-// learned frames: the CNN's input, plane 0 as the gate leaves it (the rays
-// that follow write plane 0 while the CNN runs)
-__global__ __launch_bounds__(256) void k_cnn_input(View v, const View* views)
-{
-    VIEW_OF(blockIdx.z);
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= V.N) return;
-    V.cnn_words[i] = V.screen[i];
-    V.cnn_coords[i] = V.coords[i];
 }
 
 // kernel.cl:342-401 raycast_fillhole (disabled in the reference, raycast.h:
@@ -1218,7 +1214,11 @@ __global__ void k_gate_reset(View v, const View* views)
 // a far pixel sends its residual holes and its far pixels to the list.  A
 // workgroup handles GATE_TILES tiles (each wave two, lane = 4 pixels) and
 // appends its CNN tiles and gate pixels with one atomic per list, so the
-// counters see few, uncontended atomics.
+// counters see few, uncontended atomics.  It also copies plane 0 as it finds
+// it (the rays that follow write it) for the CNN to read while they run.
+// Reads in a serial chain of eight words, with four more for a hole's quad,
+// took 24 us at 1920x1024 and the copy by itself 17; all reads together and
+// the quads from a ballot 34 for both (four learned frames 2572 -> 2505 us).
 constexpr int GATE_TILES = 8;
 __global__ __launch_bounds__(256) void k_gate(View v, const View* views, int max_cnn)
 {
@@ -1233,22 +1233,45 @@ __global__ __launch_bounds__(256) void k_gate(View v, const View* views, int max
     const uint32_t max_tiles = (uint32_t)n_tiles;
     const int fx = (res_x / 16) * 16, fy = (res_y / 16) * 16;
     const bool depth_gate = V.gate_depth > 0.0f;
+    // the wave's pixels, read together; their copy is the CNN's input
+    uint32_t w[2][4];
+    float4 c[2][4];
+    uint32_t in = 0;  // bit 4 h + j
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int h = k >> 2, j = k & 3, t = blockIdx.x * GATE_TILES + wave * 2 + h, i = lane + 64 * j;
+        const int x = (t % tiles_x) * 16 + (i & 15), y = (t / tiles_x) * 16 + (i >> 4);
+        w[h][j] = 0u;
+        c[h][j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (t >= n_tiles || x >= res_x || y >= res_y) continue;
+        in |= 1u << k;
+        w[h][j] = V.screen[(size_t)y * res_x + x];
+        c[h][j] = V.coords[(size_t)y * res_x + x];
+    }
     // per pixel: residual hole; far reprojected pixel outside the rectangle
     unsigned long long m[2][4], mp[2][4];
+#pragma unroll
     for (int h = 0; h < 2; h++) {
         const int lt = wave * 2 + h, t = blockIdx.x * GATE_TILES + lt;
         uint32_t n = 0, nf = 0;
+#pragma unroll
         for (int j = 0; j < 4; j++) {
             const int i = lane + 64 * j;
             const int x = (t % tiles_x) * 16 + (i & 15), y = (t / tiles_x) * 16 + (i >> 4);
-            const bool in = t < n_tiles && x < res_x && y < res_y;
+            const bool inside = (in >> (4 * h + j)) & 1u;
             const size_t o = (size_t)y * res_x + x;
-            const uint32_t w = in ? V.screen[o] : HOLE;
+            if (inside) {
+                V.cnn_words[o] = w[h][j];
+                V.cnn_coords[o] = c[h][j];
+            }
             const bool in_rect = x >= V.add_x && x < V.add_x + V.ext_x && y >= V.add_y && y < V.add_y + V.ext_y;
-            bool hole = in && w == HOLE && !in_rect;
-            if (hole && x < fx && y < fy && quad_is_hole(V.screen, res_x, x & ~1, y & ~1))
-                hole = false;  // in the hole list
-            const bool far = depth_gate && in && w != HOLE && !in_rect && V.coords[o].w > V.gate_depth;
+            const bool empty = inside && w[h][j] == HOLE;
+            // all four pixels of its 2x2 quad (lanes q, q + 1, q + 16, q + 17)
+            // empty, in a full 16x16 block: in the hole list
+            const unsigned long long quad = __ballot(empty) >> (lane & ~17);
+            const bool listed = x < fx && y < fy && (quad & 0x30003ull) == 0x30003ull;
+            const bool hole = empty && !in_rect && !listed;
+            const bool far = depth_gate && inside && w[h][j] != HOLE && !in_rect && c[h][j].w > V.gate_depth;
             m[h][j] = __ballot(hole);
             mp[h][j] = __ballot(far);
             n += (uint32_t)__popcll(m[h][j]);
@@ -2655,8 +2678,6 @@ static int learned_body(svo_ctx* c, svo_cnn* cnn, const svo_frame_params* p, int
     hipLaunchKernelGGL(k_gate_reset, dim3(1), dim3(1), 0, c->stream, v, (const View*)nullptr);
     hipLaunchKernelGGL(k_gate, dim3((unsigned)((tiles + GATE_TILES - 1) / GATE_TILES)), dim3(256), 0, c->stream, v,
                        (const View*)nullptr, max_cnn_holes);
-    hipLaunchKernelGGL(k_cnn_input, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0, c->stream, v,
-                       (const View*)nullptr);
     HIPCHECK(hipGetLastError());
     c->cnn_input = true;
     // The CNN reads only its input planes and writes only d_cnn_out, so it
@@ -3137,8 +3158,6 @@ static int batch_frame(svo_batch* b, const svo_frame_params* params, svo_cnn* cn
         hipLaunchKernelGGL(k_gate_reset, dim3(1, (unsigned)n), dim3(1), 0, b->stream, dummy, (const View*)dv);
         hipLaunchKernelGGL(k_gate, dim3((max_gate_tiles + GATE_TILES - 1) / GATE_TILES, (unsigned)n), dim3(256), 0,
                            b->stream, dummy, (const View*)dv, max_cnn_holes);
-        hipLaunchKernelGGL(k_cnn_input, dim3((b->maxN + 255) / 256, 1, (unsigned)n), dim3(256), 0, b->stream, dummy,
-                           (const View*)dv);
         HIPCHECK(hipGetLastError());
         for (auto* c : b->views) c->cnn_input = true;
         if (cnn) {  // all views' CNN tiles in one launch on the batch's second stream, alongside the rays
@@ -3150,7 +3169,7 @@ static int batch_frame(svo_batch* b, const svo_frame_params* params, svo_cnn* cn
             HIPCHECK(hipEventRecord(b->cnn_join, b->cnn_stream));
         }
     }
-    hipLaunchKernelGGL(k_view_first, dim3(1), dim3(1), 0, b->stream, (const View*)dv, n, b->d_first,
+    hipLaunchKernelGGL(k_view_first, dim3(1), dim3(64), 0, b->stream, (const View*)dv, n, b->d_first,
                        (uint32_t*)nullptr);
     HIPCHECK(hipGetLastError());
     RC(launch_rays_v(c0, b->stream, dummy, dv, b->d_first, n, b->d_queue, b->seq));
