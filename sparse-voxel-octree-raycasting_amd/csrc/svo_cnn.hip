@@ -194,7 +194,7 @@ __device__ __forceinline__ void conv_dw(const bf16* __restrict__ X, const bf16* 
             // past the slice: the last step's addresses again, and zeros
             const bool in = k0 + 16 * u < ke;
             const int p = min(k0 + 16 * u, ke - 16) + kq;
-            const bf16* za = dz + p * COUT;
+            const bf16* za = dz + (size_t)p * COUT;
             for (int m = 0; m < MT; m++) {
                 s4v v;
                 for (int j = 0; j < 4; j++) v[j] = (short)za[j * COUT + m * 16];
@@ -204,7 +204,7 @@ __device__ __forceinline__ void conv_dw(const bf16* __restrict__ X, const bf16* 
             // and only the pixel before and the one after can be outside it
             const int y = p / W + dy, x = p % W;
             const bool in_y = in && y >= 0 && y < H, in_l = in_y && x > 0, in_r = in_y && x + 4 < W;
-            const bf16* xa = xb + (min(max(y, 0), H - 1) * W + x) * CIN;
+            const bf16* xa = xb + (size_t)(min(max(y, 0), H - 1) * W + x) * CIN;
             const bf16* xl = xa - (x > 0 ? CIN : 0);
             const bf16* xr = xa + (x + 4 < W ? 4 : 3) * CIN;
             for (int n = 0; n < NT; n++) {
