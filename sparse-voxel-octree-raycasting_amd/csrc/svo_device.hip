@@ -219,8 +219,8 @@ struct Ray {
     int rek, lod, sxyz;
     int qx, qy, qz;  // ray_test: ix, iy, iz >> rek
     // the last step: changed position bits, their XOR, its level, whether it
-    // was taken as two trips
-    uint32_t any, xd, fuse;
+    // was taken as two trips, whether it switched the LOD
+    uint32_t any, xd, fuse, lod_up;
     int rek0;
     uint32_t node, lroot;
     uint32_t ni, st;  // ray_test: child index of the ray's cell, ST_* state
@@ -506,8 +506,8 @@ __device__ __forceinline__ void ray_step(Ray& r, const RayArgs& a, const uint32_
     const int base = max(tm + 1 - (int)fuse, rek);
     r.node = STK(base);
     r.rek = base;
-    // LOD switch, on pops only (kernel.cl:209; a far exit does not pop, but
-    // its LOD is not used again)
+    // LOD switch, on pops only (kernel.cl:209); ray_step_rules takes it back
+    // where it finds no pop
     const uint32_t l = opaque(r.dist > r.lodsw ? pop : 0u);
     r.lodsw = __builtin_amdgcn_ldexpf(r.lodsw, (int)l);
     r.lod += (int)l;
@@ -519,6 +519,7 @@ __device__ __forceinline__ void ray_step(Ray& r, const RayArgs& a, const uint32_
     r.xd = xd;
     r.rek0 = rek;
     r.fuse = fuse;
+    r.lod_up = l;
     ray_test(r, (hit << 1) | opaque(odd != 0u ? ST_RULES : 0u));
 }
 
@@ -533,6 +534,12 @@ __device__ __forceinline__ void ray_step_rules(Ray& r, const RayArgs& a, const u
     const bool far = r.dist > RAY_FAR;
     const bool pop = !far && (xm >> r.rek0) != 0u;
     const int nr = pop ? 32 - __builtin_clz(xm) : r.rek0;
+    // bit D of the XOR without a bit from rek0 to D-1 (a middle plane and a
+    // quarter plane crossed on an edge), and the far exit, are no pops
+    if (!pop) {
+        r.lod -= (int)r.lod_up;
+        r.lodsw = __builtin_amdgcn_ldexpf(r.lodsw, -(int)r.lod_up);
+    }
     if ((chg >> (nr + 1)) != 0u) r.lim = 0;
     const bool fuse = pop && r.lim != 0 && !ycross && (chg >> nr) == 0u && guard + 2u <= SVO_MAX_RAY_ITERS;
     const bool hit = fuse && nr <= r.lod;
