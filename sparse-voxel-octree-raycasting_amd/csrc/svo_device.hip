@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "svo_ctx.h"
+#include "svo_hostmem.h"
 #include "svo_internal.h"
 
 #define HOLE 0xffffff00u
@@ -3245,20 +3246,6 @@ extern "C" int svo_host_free(void* p)
     return SVO_OK;
 }
 
-// the device address of `bytes` of pinned host memory at p, or null when p is
-// anything else (or pinned for another device, or not word-aligned)
-static uint32_t* host_writable(const svo_ctx* c, void* p, size_t bytes)
-{
-    hipPointerAttribute_t a, z;
-    if (((uintptr_t)p & 3u) == 0 && hipPointerGetAttributes(&a, p) == hipSuccess && a.type == hipMemoryTypeHost &&
-        a.device == c->device && a.devicePointer &&
-        hipPointerGetAttributes(&z, (char*)p + bytes - 1) == hipSuccess && z.type == hipMemoryTypeHost &&
-        (char*)z.devicePointer - (char*)a.devicePointer == (ptrdiff_t)bytes - 1)
-        return (uint32_t*)a.devicePointer;
-    (void)hipGetLastError();
-    return nullptr;
-}
-
 extern "C" int svo_read_image_async(svo_ctx* c, uint32_t* dst)
 {
     RC(need_frame(c));
@@ -3279,7 +3266,7 @@ extern "C" int svo_read_image_async(svo_ctx* c, uint32_t* dst)
         HIPCHECK(hipMemset(c->image_buf[1], 0, 4 * c->N));
     }
     const int s = c->d_image == c->image_buf[1] ? 1 : 0;
-    uint32_t* out = host_writable(c, dst, 4 * c->N);
+    uint32_t* out = svo_host_writable(c->device, dst, 4 * c->N);
     // the kernel on the CNN's stream (idle in frames without a CNN, and a
     // learned frame's CNN starts later than the copy of the one before ends):
     // a stream of its own would be one more on the few hardware queues
