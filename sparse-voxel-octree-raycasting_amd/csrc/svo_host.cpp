@@ -19,8 +19,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -411,7 +411,7 @@ size_t first_bad_block(const Validator& proto, const std::vector<BlockRef>& bloc
     for (size_t t = 0; t < extra; t++) {
         try {
             th[t] = std::thread(work);
-        } catch (const std::system_error&) {  // no thread to be had: fewer
+        } catch (const std::exception&) {  // no thread, or no memory for its state: fewer
             break;
         }
     }
