@@ -431,7 +431,11 @@ int svo_cnn_get_params(svo_cnn* cnn, float* dst, size_t count);
 int svo_cnn_set_params(svo_cnn* cnn, const float* src, size_t count);
 /* x: [batch][h][w][16] bf16 bit patterns (h, w multiples of 8), zero
  * "same" padding at crop borders; out: [batch][h][w][16] float (channels
- * 0..2 = RGB in 0..1). */
+ * 0..2 = RGB in 0..1).  The network keeps its workspace for the largest batch
+ * so far: 288 bytes of device memory per pixel; once it has made gradients
+ * (svo_cnn_gradients, svo_cnn_train_step) 240 more, and partial sums of 108 KB
+ * per crop and 2 bytes per pixel up to 2,427 crops, beyond them 36 KB per crop
+ * and half a byte per pixel. */
 int svo_cnn_forward(svo_cnn* cnn, const uint16_t* x, int batch, int h, int w, float* out);
 /* loss = sum mask*(out-target)^2 / (3*sum mask) over RGB; writes the
  * gradient of every parameter (same layout as the parameter vector). */

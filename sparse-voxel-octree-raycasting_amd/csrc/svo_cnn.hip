@@ -946,11 +946,14 @@ struct svo_cnn {
     bf16 *wbf = nullptr, *wflip = nullptr;
     float* h_grads = nullptr;  // pinned: kParams gradients and the loss
     int step = 0;
-    // activation workspace for the current batch size
+    // activation workspace for the current batch size: 288 bytes per pixel
     size_t cap_pix = 0;
     bf16* x0 = nullptr;    // [pix][16]
     bf16* y[3] = {};       // [pix][32]
     float* out = nullptr;  // [pix][16]
+    // and what gradients need beside it, allocated by the first call that
+    // makes them: 240 bytes per pixel
+    size_t cap_grad = 0;
     bf16* dz[4] = {};      // [pix][32], the last layer's [pix][16]
     float* target = nullptr;
     float* mask = nullptr;
@@ -979,36 +982,50 @@ struct svo_cnn {
             return svo_fail(SVO_ERR_HIP, "%s failed: %s", #expr, hipGetErrorString(_e)); \
     } while (0)
 
-static void free_ws(svo_cnn* n)
+static void free_forward_ws(svo_cnn* n)
 {
     (void)hipFree(n->x0);
     for (auto& p : n->y) (void)hipFree(p);
     (void)hipFree(n->out);
-    for (auto& p : n->dz) (void)hipFree(p);
-    (void)hipFree(n->target);
-    (void)hipFree(n->mask);
     n->x0 = nullptr;
     for (auto& p : n->y) p = nullptr;
     n->out = nullptr;
-    for (auto& p : n->dz) p = nullptr;
-    n->target = n->mask = nullptr;
     n->cap_pix = 0;
 }
 
-static int ensure_ws(svo_cnn* n, size_t pix)
+static void free_grad_ws(svo_cnn* n)
 {
-    if (pix <= n->cap_pix) return SVO_OK;
-    free_ws(n);
-    bool ok = hipMalloc(&n->x0, pix * 16 * 2) == hipSuccess && hipMalloc(&n->y[0], pix * 32 * 2) == hipSuccess &&
-              hipMalloc(&n->y[1], pix * 32 * 2) == hipSuccess && hipMalloc(&n->y[2], pix * 32 * 2) == hipSuccess &&
-              hipMalloc(&n->out, pix * 16 * 4) == hipSuccess &&
-              hipMalloc(&n->target, pix * 3 * 4) == hipSuccess && hipMalloc(&n->mask, pix * 4) == hipSuccess;
-    for (int l = 0; l < 4; l++) ok = ok && hipMalloc(&n->dz[l], pix * kCout[l] * 2) == hipSuccess;
-    if (!ok) {
-        free_ws(n);
-        return svo_fail(SVO_ERR_NOMEM, "CNN workspace for %zu pixels", pix);
+    for (auto& p : n->dz) (void)hipFree(p);
+    (void)hipFree(n->target);
+    (void)hipFree(n->mask);
+    for (auto& p : n->dz) p = nullptr;
+    n->target = n->mask = nullptr;
+    n->cap_grad = 0;
+}
+
+// the workspace of a forward over pix pixels, and of its gradients
+static int ensure_ws(svo_cnn* n, size_t pix, bool grads)
+{
+    if (pix > n->cap_pix) {
+        free_forward_ws(n);
+        bool ok = hipMalloc(&n->x0, pix * 16 * 2) == hipSuccess && hipMalloc(&n->out, pix * 16 * 4) == hipSuccess;
+        for (auto& p : n->y) ok = ok && hipMalloc(&p, pix * 32 * 2) == hipSuccess;
+        if (!ok) {
+            free_forward_ws(n);
+            return svo_fail(SVO_ERR_NOMEM, "CNN workspace for %zu pixels", pix);
+        }
+        n->cap_pix = pix;
     }
-    n->cap_pix = pix;
+    if (grads && pix > n->cap_grad) {
+        free_grad_ws(n);
+        bool ok = hipMalloc(&n->target, pix * 3 * 4) == hipSuccess && hipMalloc(&n->mask, pix * 4) == hipSuccess;
+        for (int l = 0; l < 4; l++) ok = ok && hipMalloc(&n->dz[l], pix * kCout[l] * 2) == hipSuccess;
+        if (!ok) {
+            free_grad_ws(n);
+            return svo_fail(SVO_ERR_NOMEM, "CNN gradient workspace for %zu pixels", pix);
+        }
+        n->cap_grad = pix;
+    }
     return SVO_OK;
 }
 
@@ -1027,7 +1044,8 @@ extern "C" int svo_cnn_destroy(svo_cnn* n)
     if (!n) return SVO_OK;
     (void)hipSetDevice(n->device);
     (void)hipStreamSynchronize(n->stream);
-    free_ws(n);
+    free_forward_ws(n);
+    free_grad_ws(n);
     for (float* p : {n->params, n->grads, n->m, n->v}) (void)hipFree(p);
     (void)hipFree(n->wbf);
     (void)hipFree(n->wflip);
@@ -1209,7 +1227,7 @@ extern "C" int svo_cnn_forward(svo_cnn* n, const uint16_t* x, int B, int H, int 
     if (rc) return rc;
     HIPCHECK(hipSetDevice(n->device));
     const size_t pix = (size_t)B * H * W;
-    rc = ensure_ws(n, pix);
+    rc = ensure_ws(n, pix, false);
     if (rc) return rc;
     HIPCHECK(hipMemcpyAsync(n->x0, x, pix * 16 * 2, hipMemcpyHostToDevice, n->stream));
     rc = cnn_forward_dev(n, B, H, W);
@@ -1230,7 +1248,7 @@ extern "C" int svo_cnn_gradients(svo_cnn* n, const uint16_t* x, const float* tar
     if (rc) return rc;
     HIPCHECK(hipSetDevice(n->device));
     const size_t pix = (size_t)B * H * W;
-    rc = ensure_ws(n, pix);
+    rc = ensure_ws(n, pix, true);
     if (rc) return rc;
     HIPCHECK(hipMemcpyAsync(n->x0, x, pix * 16 * 2, hipMemcpyHostToDevice, n->stream));
     HIPCHECK(hipMemcpyAsync(n->target, target, pix * 3 * 4, hipMemcpyHostToDevice, n->stream));
@@ -1280,7 +1298,7 @@ extern "C" int svo_cnn_train_step(svo_cnn* n, svo_ctx* warp, svo_ctx* full, cons
     if (n_crops <= 0 || n_crops > 256 || crop < 16 || crop % 8 || crop > warp->res_x || crop > warp->res_y)
         return svo_fail(SVO_ERR_ARG, "bad crop batch %d x %d", n_crops, crop);
     HIPCHECK(hipSetDevice(n->device));
-    int rc = ensure_ws(n, (size_t)n_crops * crop * crop);
+    int rc = ensure_ws(n, (size_t)n_crops * crop * crop, true);
     if (rc) return rc;
     if (n->max_origins < n_crops) {
         (void)hipFree(n->origins);
@@ -1388,7 +1406,7 @@ int cnn_fill_tiles(svo_cnn* n, svo_ctx* c, const svo_frame_params* p, const uint
         a.v = tile_view(c, p, tile_list, tile_count, max_tiles);
         return launch_tiles(a, max_tiles, n->n_cu, stream, grid);
     }
-    int rc = ensure_ws(n, (size_t)max_tiles * 576);
+    int rc = ensure_ws(n, (size_t)max_tiles * 576, false);
     if (rc) return rc;
     hipStream_t keep = n->stream;
     n->stream = stream;  // run on the frame's stream
