@@ -160,8 +160,9 @@ int svo_read(svo_ctx* ctx, int buf, size_t byte_ofs, size_t bytes, void* dst);
  * 425-455); calls that write part of the image or none keep the buffer.
  * dst should be pinned host memory (svo_host_alloc) for the copy to run
  * asynchronously; it holds the image once svo_sync returns.  A buffer is
- * reused two frames later, after its copy has completed.  For a view of a
- * batch, call svo_batch_sync first. */
+ * reused two frames later, after its copy has completed.  A learned frame's
+ * CNN runs behind the copy of the image before it into pinned memory.  For a
+ * view of a batch, call svo_batch_sync first. */
 int svo_read_image_async(svo_ctx* ctx, uint32_t* dst);
 /* Pinned (page-locked) host memory for svo_read_image_async destinations,
  * and its release.  No reference counterpart (ocl_copy_to_host, ocl.h:215,
@@ -346,10 +347,11 @@ int svo_set_long_first(svo_ctx* ctx, int long_trips);
  * no earlier frame to overlap, and its own rays finish sooner without one.
  * Defaults: 3 sets (until the first svo_set_pretrace a frame whose
  * predecessor was read with svo_read_image_async uses two of them, which
- * leaves a hardware queue to the image copies), long_trips 1, 1 workgroup per CU, no split,
- * only_queued 1, predict 2, whole_trips 0, queue_skip 3.  A primary ray depends
- * only on the camera, the pixel and the octree (kernel.cl:594-694,
- * :846-942): results do not depend on these settings.  HIP maps streams onto
+ * leaves a hardware queue to the image copies; in a process whose other
+ * streams shift the queues three can be the faster number then), long_trips
+ * 1, 1 workgroup per CU, no split, only_queued 1, predict 2, whole_trips 0,
+ * queue_skip 3.  A primary ray depends only on the camera, the pixel and the
+ * octree (kernel.cl:594-694, :846-942): results do not depend on these settings.  HIP maps streams onto
  * at most GPU_MAX_HW_QUEUES hardware queues (4 unless the environment sets
  * it before the first HIP call); pretraces whose streams share one run one
  * after the other.

@@ -511,9 +511,10 @@ __global__ __launch_bounds__(256) void k_cnn_apply(const uint32_t* __restrict__ 
 // beside it on one device: 276.5 us with nine reads per M-tile and each
 // layer's weights staged in LDS, 203 with the sweep and the resident weights,
 // 178 with the next row's fragments read behind a row's first MFMAs, 169 with
-// layer 4's RGB stored from its registers and the crop fetched ahead.  At 169
-// the matrix cores are busy 39 % of the time; two waves per SIMD (LDS and
-// registers both allow no more) leave each other's stalls uncovered.
+// layer 4's RGB stored from its registers and the crop fetched ahead.  The
+// matrix cores are then busy in 42 % of the cycles (counters); two waves per
+// SIMD (LDS and registers both allow no more) leave each other's stalls
+// uncovered.
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 
 // 32-channel buffers: rows of TILE_PITCH pixels of 64 bytes; the 16-byte

@@ -1434,10 +1434,16 @@ extern "C" int svo_create(svo_ctx** out, int device)
     if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
         c->n_cu = prop.multiProcessorCount;
     // The CNN tile kernel beside the ray launch: three quarters of the CUs.
-    // Learned frames back to back / each synced, us per frame: 1920x1024
-    // depth 11 at half 753 / 734, three quarters 636 / 663, all 626 / 666, two
-    // per CU 630 / 664; 1280x720 depth 10 710 / 780, 685 / 815, 700 / 832,
-    // 688 / 832; 640x480 314 / 445, 298 / 455, 295 / 470, 295 / 493.
+    // With more workgroups the CNN ends earlier and the rays beside it later.
+    // Issued back to back, more is faster at every size; synced each, a frame
+    // of about a megapixel is as long as its rays and loses, a larger one as
+    // long as its CNN.  Learned frames back to back / each synced, us per
+    // frame, at half, three quarters, all of the CUs: 640x480 depth 9 473 / 406,
+    // 465 / 412, 458 / 412; 1280x720 depth 10 844 / 827, 799 / 843, 783 / 856;
+    // 1361x763 947 / 966, 899 / 980, 888 / 1007; 1920x1024 depth 11 997 / 741,
+    // 893 / 675, 858 / 673; 2560x1440 1583 / 1174, 1379 / 970, 1310 / 917;
+    // 3840x2160 3235 / 2457, 2719 / 1983, 2546 / 1802.  Three quarters costs
+    // the synced megapixel frame 1.5-2% and takes most of the rest.
     c->cnn_overlap_wgs = std::max(1, c->n_cu * 3 / 4);
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess &&
               hipStreamCreateWithFlags(&c->cnn_stream, hipStreamNonBlocking) == hipSuccess;
@@ -2554,9 +2560,14 @@ static int pretrace(svo_ctx* c, const svo_frame_params* p, int gate_max)
     // By default three sets, and two while the images are read back: then the
     // copies need a hardware queue too (four, one of them the frames' own),
     // and behind a pretrace's rays they would hold up the frame that waits for
-    // the image buffer.  Frames with every image read, three sets / two:
-    // 1920x1024 497 / 438 us, 1361x763 605 / 507, 1280x720 cave 298 / 269,
-    // learned 1920x1024 725 / 660; without reading 1361x763 340 / 460.
+    // the image buffer.  What shares a queue depends on the streams the
+    // process made before the context's.  Frames with every image read, three
+    // sets / two, us per frame, with 0, 1, 2, 3 other streams alive: 1920x1024
+    // 541 / 571, 599 / 763, 581 / 447, 534 / 432; 1361x763 668 / 595, 712 / 968,
+    // 680 / 507, 647 / 509; 1280x720 cave 289 / 316, 331 / 380, 344 / 289,
+    // 282 / 239.  With one, svo_set_pretrace with three sets is the faster one.
+    // Without reading, three / two: 1361x763 599 / 573, 599 / 569, 596 / 465,
+    // 341 / 464.
     const int s = (int)(c->pre_frames % (uint32_t)(c->pre_auto && c->image_reads ? 2 : c->pre_sets));
     const uint32_t id = c->pre_frames + 1u;
     const bool pred = predict_ready(c, p);
@@ -3267,9 +3278,11 @@ extern "C" int svo_read_image_async(svo_ctx* c, uint32_t* dst)
     }
     const int s = c->d_image == c->image_buf[1] ? 1 : 0;
     uint32_t* out = svo_host_writable(c->device, dst, 4 * c->N);
-    // the kernel on the CNN's stream (idle in frames without a CNN, and a
-    // learned frame's CNN starts later than the copy of the one before ends):
-    // a stream of its own would be one more on the few hardware queues
+    // The kernel runs on the CNN's stream: a stream of its own would be one
+    // more on the few hardware queues.  A learned frame's CNN queues behind the
+    // copy of the image before: at 1920x1024 it could start 118 us into the
+    // frame and the copy takes 147.  Learned frames not read / read, three
+    // pretrace sets, us per frame: 1920x1024 860 / 918, 1361x763 925 / 1015.
     hipStream_t st = out ? c->cnn_stream : c->copy_stream;
     HIPCHECK(hipEventRecord(c->image_ready, c->stream));
     HIPCHECK(hipStreamWaitEvent(st, c->image_ready, 0));
