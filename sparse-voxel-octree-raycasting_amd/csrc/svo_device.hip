@@ -40,7 +40,7 @@ namespace {
 
 constexpr int RAY_BLOCK = 256;
 // Iterations (a step and a descend each) per wave-uniform exit check.
-// Measured on one box (lone ray of 3,589 trips, with 68 us of launch / 1920x1024
+// Measured on one device (lone ray of 3,589 trips, with 68 us of launch / 1920x1024
 // depth-11 flights: 8 warp frames, 2 full frames): 2: 570 us / 4.51 ms /
 // 1.57 ms; 4: 512 / 4.37 / 1.54; 8: 509 / 4.31 / 1.52; 16: 501 / 4.28 / 1.53.
 #ifndef SVO_TRIP_UNROLL
